@@ -685,11 +685,11 @@ class HipBackend : public Backend {
     const float* k = in(op.in[1], c);
     const float* v = in(op.in[2], c);
     const int idx = static_cast<int>(&op - c.graph->ops.data());
-    if (prepared_ && fuse_attn_[idx] && !capturing_ && T > 1) {
+    if (prepared_ && fuse_attn_[idx] && T > 1) {
       attn_ = {idx, q, k, v, out(op.out[0], c), T, c.pos0, nh, nkv, hd, l.k, l.v, mc, rc, rs};
       return;  // the next op (the o projection) runs it
     }
-    if (capturing_)  // the replayed step reads its position from device memory
+    if (capturing_ && T == 1)  // the replayed step reads its position from device memory (a prefill graph's is fixed)
       check(elmh_attention_step_dev(ctx_, q, k, v, out(op.out[0], c), pos_dev_, nh, nkv, hd, l.k, l.v, mc, rc, rs), op);
     else
       check(elmh_attention_dev(ctx_, q, k, v, out(op.out[0], c), T, c.pos0, nh, nkv, hd, l.k, l.v, mc, rc, rs), op);
