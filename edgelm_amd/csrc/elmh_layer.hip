@@ -1106,6 +1106,419 @@ __global__ __launch_bounds__(256) void attention_prefill64_kernel(
   }
 }
 
+// Chunks of a prompt (T > 1) at any head size: one 256-thread workgroup per kv head and R rows, a row being one (query
+// token, head of the kv head's group) pair, tokens slowest, so the group's heads share every key and value read. The
+// same float operations in the same order as attention_kernel (cpu::attention). What bounds it is the vector ALU: an
+// unfused multiply and add per (row, position, dim) in the scores and in the output sums, with no other form that rounds
+// alike (f32 MFMA outer products give the same products, but they and the adds took 3.8-4.4 clocks per 64 together where
+// multiply and add on the VALU take 4.3: no gain).
+//  - scores: a lane holds one position, a wave 64 positions of a 256-position tile. Its 64 key rows pass through a 4 KB
+//    piece of LDS of its own, 16 dims at a time, by DMA (the 16-byte chunk u of row r in slot u ^ (r / 4 % 4), so that 16
+//    lanes reading chunk u hit every bank once), into 16 registers; the next piece is requested before the multiplies. A
+//    row's 16 query dims lie in 16 lanes of one register and are broadcast by the multiply itself (row_bcast), four
+//    chains per row: R * 64 multiplies and adds per 16 dims against R + 4 LDS reads, and no barrier in the loop.
+//  - softmax: 256 / R lanes per row; the exponentials' table in LDS; the in-order sum in every lane of the row at once.
+//  - output: a lane holds one dim of R / (2 RS) rows (a wave 32 dims, its two halves different rows; RS = 2 splits the
+//    rows over two pairs of waves where two waves cover the dims); values come straight from the cache, 16 positions per
+//    batch, the next batch in flight; p_j = e_j * inv of 16 positions lies in 16 lanes and is broadcast by the multiply.
+//    Positions that only some of the rows see are masked (a later token's value may be anything), the others are not.
+// 32 heads over 8 kv heads, head size 128, 256 tokens at 256 cached positions: 73 us with the append against 800 us with one workgroup per
+// (token, head) (attention_kernel), which read the keys and values again for every row and ran each row's chains on one wave.
+// LDS (dynamic): scores [R][scs], 256 floats that reads ahead may touch, key pieces [4][64][16], queries [R][16 ceil(hd/16)].
+template <int R, int RS>
+__global__ __launch_bounds__(256) void attention_rows_kernel(const float* __restrict__ q, float* __restrict__ out,
+                                                             const float* __restrict__ kc, const float* __restrict__ vc,
+                                                             int pos0, int T, int grp, int n_kv, int hd, int max_ctx, int scs,
+                                                             const float* __restrict__ rcos, const float* __restrict__ rsin,
+                                                             int8_t* __restrict__ xq, float* __restrict__ xd, int Tpad) {
+  constexpr int LPR = 256 / R, RPL = R / (2 * RS);
+  extern __shared__ __align__(16) float lds[];
+  __shared__ uint64_t etab[32];
+  __shared__ float inv_s[R];
+  float* const sc = lds;
+  float* const kb = sc + R * scs + 256;
+  float* const qb = kb + 4 * 1024;
+  const int hdq = (hd + 15) & ~15, hd4 = hd >> 2, h2 = hd >> 1;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kvh = blockIdx.x, nrows = T * grp, qd = n_kv * grp * hd;
+  // the last rows (the longest) first: the short ones fill in behind them
+  const int r0 = (gridDim.y - 1 - blockIdx.y) * R;
+  const int t_first = r0 / grp, t_last = min(r0 + R - 1, nrows - 1) / grp;
+  const int nmin = pos0 + t_first + 1, nmax = pos0 + t_last + 1;  // positions every row sees, and any row sees
+  const float* const kh = kc + (int64_t)kvh * max_ctx * hd;
+  const float* const vh = vc + (int64_t)kvh * max_ctx * hd;
+  if (tid < 32) etab[tid] = elm_exp2_tab(tid);
+
+  const int nst = hdq >> 4;
+  float* const kw = kb + w * 1024;
+  const unsigned kw_lds = (unsigned)(size_t)(LdsBytes)(unsigned char*)kw;
+  // 16 dims of the wave's 64 key rows from position `base` on (positions past nmax repeat the last one, dims past hd the
+  // last four)
+  auto request = [&](int base, int st) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * i + (lane >> 2), ch = (lane & 3) ^ ((r >> 2) & 3);
+      dma16s(kh, (uint32_t)((min(base + r, nmax - 1) * hd4 + min(4 * st + ch, hd4 - 1)) << 4), kw_lds + i * 1024);
+    }
+  };
+  if (64 * w < nmax) request(64 * w, 0);
+
+  // the rows' queries, rotated (pairs (i, i + hd / 2)), into LDS
+  for (int f = tid; f < R * h2; f += 256) {
+    const int r = f / h2, i = f - r * h2, rr = min(r0 + r, nrows - 1), t = rr / grp, h = kvh * grp + rr - t * grp;
+    const float* const qs = q + (int64_t)t * qd + h * hd;
+    const float a = qs[i], b = qs[i + h2];
+    float x = a, y = b;
+    if (rcos) {
+      const float c = rcos[(int64_t)(pos0 + t) * h2 + i], s = rsin[(int64_t)(pos0 + t) * h2 + i];
+      x = a * c - b * s;
+      y = b * c + a * s;
+    }
+    qb[r * hdq + i] = x;
+    qb[r * hdq + i + h2] = y;
+  }
+  lds_barrier();
+
+  // scores
+  const float scale = 1.0f / sqrtf((float)hd);
+  for (int base = 64 * w; base < nmax; base += 256) {
+    float acc[R][4];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[r][c] = 0.f;
+    for (int st = 0; st < nst; ++st) {
+      wait_vm<0>();  // this wave's piece has landed
+      asm volatile("" ::: "memory");
+      v4f k[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        k[u] = *reinterpret_cast<const v4f*>(kw + lane * 16 + ((u ^ ((lane >> 2) & 3)) << 2));
+      float qr[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) qr[r] = qb[r * hdq + 16 * st + (lane & 15)];
+      // the piece is in registers before the next one overwrites it
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      asm volatile("" : "+v"(k[0]), "+v"(k[1]), "+v"(k[2]), "+v"(k[3])::"memory");
+      if (st + 1 < nst)
+        request(base, st + 1);
+      else if (base + 256 < nmax)
+        request(base + 256, 0);
+#define ELM_SCORE_STEP(n)                                                                       \
+  _Pragma("unroll") for (int r = 0; r < R; ++r) acc[r][(n) & 3] = acc[r][(n) & 3] + row_bcast<n>(qr[r]) * k[(n) >> 2][(n) & 3];
+#define ELM_SCORE_STEP4(u) ELM_SCORE_STEP(4 * (u)) ELM_SCORE_STEP(4 * (u) + 1) ELM_SCORE_STEP(4 * (u) + 2) ELM_SCORE_STEP(4 * (u) + 3)
+      const int nd4 = min(4, hd4 - 4 * st);  // 4 except in the last piece of a head size that 16 does not divide
+      if (nd4 == 4) {
+        ELM_SCORE_STEP4(0) ELM_SCORE_STEP4(1) ELM_SCORE_STEP4(2) ELM_SCORE_STEP4(3)
+      } else {
+        ELM_SCORE_STEP4(0)
+        if (nd4 > 1) { ELM_SCORE_STEP4(1) }
+        if (nd4 > 2) { ELM_SCORE_STEP4(2) }
+      }
+#undef ELM_SCORE_STEP4
+#undef ELM_SCORE_STEP
+    }
+    if (base + lane < nmax) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        sc[r * scs + base + lane] = ((acc[r][0] + acc[r][1]) + (acc[r][2] + acc[r][3])) * scale;
+    }
+  }
+  __syncthreads();
+
+  // softmax: LPR lanes per row; e_j up to the row's last position, +0.0 from there to the next multiple of 16 of nmax
+  const int n16 = (nmax + 15) & ~15;
+  {
+    const int r = tid / LPR, l = tid % LPR, nr = pos0 + min(r0 + r, nrows - 1) / grp + 1;
+    float* const row = sc + r * scs;
+    float mx = -INFINITY;
+    for (int j = l; j < nr; j += LPR) mx = fmaxf(mx, row[j]);
+    mx = fmaxf(mx, dpp_f<kDppQuadXor1>(mx));
+    mx = fmaxf(mx, dpp_f<kDppQuadXor2>(mx));
+    mx = fmaxf(mx, dpp_f<kDppHalfMirror>(mx));
+    mx = fmaxf(mx, dpp_f<kDppRowMirror>(mx));
+    if (LPR > 16) mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    if (LPR > 32) mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    for (int j = l; j < n16; j += LPR) row[j] = j < nr ? elm_expf_tab(row[j] - mx, etab) : 0.f;
+    // the row's lanes share a wave: their writes are ordered before its reads below
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    float sum = 0.f;
+    for (int g0 = 0; g0 < n16; g0 += 256) sum = ordered_sum256(row + g0, min(16, (n16 - g0) >> 4), sum);
+    if (l == 0) inv_s[r] = 1.0f / sum;
+  }
+  __syncthreads();
+
+  // output sums
+  constexpr int DW = 4 / RS;  // waves side by side over the dims
+  const int rs = w / DW, half = lane >> 5, rw = rs * (R / RS) + half * RPL;
+  float inv[RPL];
+  int nr[RPL];
+#pragma unroll
+  for (int i = 0; i < RPL; ++i) {
+    inv[i] = inv_s[rw + i];
+    nr[i] = pos0 + min(r0 + rw + i, nrows - 1) / grp + 1;
+  }
+  for (int d0 = 32 * (w % DW); d0 < hd; d0 += 32 * DW) {
+    const int dim = d0 + (lane & 31);
+    const float* const vd = vh + min(dim, hd - 1);
+    float acc[RPL], va[16], vb[16];
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) acc[i] = 0.f;
+    auto load = [&](int j0, float (&v)[16]) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = vd[(int64_t)min(j0 + u, nmax - 1) * hd];
+    };
+#define ELM_OUT_STEP(n)                                                            \
+  _Pragma("unroll") for (int i = 0; i < RPL; ++i) {                                \
+    const float pv = row_bcast<n>(p[i]) * v[n];                                    \
+    acc[i] = acc[i] + (full || j0 + (n) < nr[i] ? pv : 0.f);                       \
+  }
+    auto batch = [&](int j0, const float (&v)[16], bool full) __attribute__((always_inline)) {
+      float p[RPL];
+#pragma unroll
+      for (int i = 0; i < RPL; ++i) p[i] = sc[(rw + i) * scs + j0 + (lane & 15)] * inv[i];
+      ELM_OUT_STEP(0) ELM_OUT_STEP(1) ELM_OUT_STEP(2) ELM_OUT_STEP(3) ELM_OUT_STEP(4) ELM_OUT_STEP(5) ELM_OUT_STEP(6)
+      ELM_OUT_STEP(7) ELM_OUT_STEP(8) ELM_OUT_STEP(9) ELM_OUT_STEP(10) ELM_OUT_STEP(11) ELM_OUT_STEP(12) ELM_OUT_STEP(13)
+      ELM_OUT_STEP(14) ELM_OUT_STEP(15)
+    };
+#undef ELM_OUT_STEP
+    const int nfull = nmin & ~15;  // whole batches that every row sees
+    load(0, va);
+    int j0 = 0;
+    for (; j0 + 32 <= nfull; j0 += 32) {
+      load(j0 + 16, vb);
+      batch(j0, va, true);
+      load(j0 + 32, va);
+      batch(j0 + 16, vb, true);
+    }
+    for (; j0 < nmax; j0 += 16) {
+      load(j0 + 16, vb);
+      if (j0 < nfull)
+        batch(j0, va, true);
+      else
+        batch(j0, va, false);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) va[u] = vb[u];
+    }
+    if (dim < hd) {
+#pragma unroll
+      for (int i = 0; i < RPL; ++i) {
+        const int rr = r0 + rw + i, t = min(rr, nrows - 1) / grp, h = kvh * grp + rr - t * grp;
+        if (rr < nrows) out[(int64_t)t * qd + h * hd + dim] = acc[i];
+        if (xq) {
+          // head size 64: the half-wave holds one 32-element block of the token's output (block 2 h or 2 h + 1), written as
+          // the next GEMM's activation fragments as attention_prefill64_kernel does (every lane of the half is here)
+          float a = fmaxf(0.f, fabsf(acc[i]));
+#pragma unroll
+          for (int m = 1; m < 32; m <<= 1) a = fmaxf(a, __shfl_xor(a, m, 64));
+          const float scl = a / 127.0f;
+          int qv;
+          elm_q8_group<1>(&acc[i], scl == 0.f ? 1.f : scl, &qv);
+          const int b = (h * hd + d0) >> 5, e = lane & 31;
+          if (rr < nrows) {
+            xq[elm_frag_offset(t, b, e >> 4, qd >> 5) + (e & 15)] = (int8_t)qv;
+            if (e == 0) xd[(int64_t)b * Tpad + t] = scl;
+          }
+        }
+      }
+    }
+  }
+}
+
+// One 1024-thread workgroup per (query token, head) at any head size: decode steps (FUSE: one token, the append inside, the
+// position possibly in device memory) and chunks of a few tokens, where attention_rows_kernel's workgroups would be too few
+// to fill the chip. The same float operations in the same order as attention_kernel (cpu::attention). Latency bounds it, so
+// every phase that is not one ordered chain is spread over 16 waves:
+//  - scores as in attention_rows_kernel: a lane per position, 64 positions per wave and 1024 per pass, 16 dims of a wave's
+//    key rows at a time through a 4 KB LDS piece of its own, the query broadcast by the multiply;
+//  - the in-order sum of the exponentials on wave 0 while the waves that will add the values request the first 64 positions;
+//  - output: a lane per dim, four batches of 16 positions in flight (one position's values are one coalesced request).
+// The step's own key (rotated) replaces its row of the piece in LDS and its value is added last from a register, as the kv
+// group's first workgroup is still writing them to the cache.
+// 32 heads over 8 kv heads, head size 128, 700 cached positions: 22 us against 44 us with attention_kernel.
+// LDS (dynamic): scores [n_cap rounded up to 16, and 256 more that reads ahead may touch], key pieces [16][64][16], query and
+// step's key [16 ceil(hd / 16)] each.
+constexpr int kStepWaves = 16;
+template <bool FUSE>
+__global__ __launch_bounds__(64 * kStepWaves) void attention_step_kernel(
+    const float* __restrict__ q, float* __restrict__ out, float* __restrict__ kc, float* __restrict__ vc, int pos0,
+    const int* __restrict__ pos_dev, int grp, int n_kv, int hd, int max_ctx, int n_cap, const float* __restrict__ rcos,
+    const float* __restrict__ rsin, const float* __restrict__ knew, const float* __restrict__ vnew) {
+  constexpr int NT = 64 * kStepWaves;
+  // every argument into scalar registers first, in one batch of loads (as the head-size-64 kernels)
+  asm volatile("" ::"s"(q), "s"(out), "s"(kc), "s"(vc), "s"(pos0), "s"(pos_dev), "s"(grp), "s"(n_kv), "s"(hd), "s"(max_ctx),
+               "s"(n_cap), "s"(rcos), "s"(rsin), "s"(knew), "s"(vnew));
+  extern __shared__ __align__(16) float lds[];
+  __shared__ uint64_t etab[32];
+  __shared__ float red[kStepWaves];
+  __shared__ float inv_s;
+  const int hdq = (hd + 15) & ~15, hd4 = hd >> 2, h2 = hd >> 1, nst = hdq >> 4;
+  float* const sc = lds;
+  float* const kb = sc + ((n_cap + 15) & ~15) + 256;
+  float* const qb = kb + kStepWaves * 1024;
+  float* const kn = qb + hdq;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kvh = blockIdx.x, h = kvh * grp + blockIdx.y, t = blockIdx.z, qd = n_kv * grp * hd;
+  // q (and the step's key) before the position has arrived
+  const float* const qs = q + (int64_t)t * qd + h * hd;
+  const int ih = tid < h2 ? tid : 0;
+  const float qa = qs[ih], qz = qs[ih + h2];
+  float ka = 0.f, kz = 0.f, va = 0.f, vz = 0.f;
+  if (FUSE) {
+    ka = knew[kvh * hd + ih];
+    kz = knew[kvh * hd + ih + h2];
+    va = vnew[kvh * hd + ih];
+    vz = vnew[kvh * hd + ih + h2];
+  }
+  // the caller keeps the position in range; stay in bounds anyway
+  const int pos = FUSE && pos_dev ? min(max(*pos_dev, 0), max_ctx - 1) : pos0 + t;
+  const int n = pos + 1, nc = FUSE ? n - 1 : n;  // positions, and those whose rows come from the cache
+  const float* const kh = kc + (int64_t)kvh * max_ctx * hd;
+  const float* const vh = vc + (int64_t)kvh * max_ctx * hd;
+  float* const kw = kb + w * 1024;
+  const unsigned kw_lds = (unsigned)(size_t)(LdsBytes)(unsigned char*)kw;
+  const int rlast = max(nc - 1, 0);
+  auto request = [&](int base, int st) {  // as attention_rows_kernel's
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * i + (lane >> 2), ch = (lane & 3) ^ ((r >> 2) & 3);
+      dma16s(kh, (uint32_t)((min(base + r, rlast) * hd4 + min(4 * st + ch, hd4 - 1)) << 4), kw_lds + i * 1024);
+    }
+  };
+  if (64 * w < n) request(64 * w, 0);
+  if (tid < 32) etab[tid] = elm_exp2_tab(tid);
+  if (tid < h2) {
+    float c = 1.f, s = 0.f;
+    if (rcos) {
+      c = rcos[(int64_t)pos * h2 + tid];
+      s = rsin[(int64_t)pos * h2 + tid];
+    }
+    qb[tid] = rcos ? qa * c - qz * s : qa;
+    qb[tid + h2] = rcos ? qz * c + qa * s : qz;
+    if (FUSE) {
+      // step 1 of cpu::attention for this token (kv_append_kernel's arithmetic)
+      const float k0 = rcos ? ka * c - kz * s : ka, k1 = rcos ? kz * c + ka * s : kz;
+      kn[tid] = k0;
+      kn[tid + h2] = k1;
+      if (blockIdx.y == 0) {
+        float* const kd = kc + ((int64_t)kvh * max_ctx + pos) * hd;
+        float* const vd = vc + ((int64_t)kvh * max_ctx + pos) * hd;
+        kd[tid] = k0;
+        kd[tid + h2] = k1;
+        vd[tid] = va;
+        vd[tid + h2] = vz;
+      }
+    }
+  }
+  lds_barrier();
+
+  // scores
+  const float scale = 1.0f / sqrtf((float)hd);
+  float mx = -INFINITY;
+  for (int base = 64 * w; base < n; base += NT) {
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int st = 0; st < nst; ++st) {
+      wait_vm<0>();
+      asm volatile("" ::: "memory");
+      if (FUSE && n - 1 - base < 64 && lane < 4) {  // the step's key in its row of the piece (lane: its 16-byte chunk)
+        const int r = n - 1 - base;
+        *reinterpret_cast<v4f*>(kw + r * 16 + ((lane ^ ((r >> 2) & 3)) << 2)) = *reinterpret_cast<const v4f*>(kn + 16 * st + 4 * lane);
+      }
+      v4f k[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        k[u] = *reinterpret_cast<const v4f*>(kw + lane * 16 + ((u ^ ((lane >> 2) & 3)) << 2));
+      const float qr = qb[16 * st + (lane & 15)];
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the piece is in registers before the next one overwrites it
+      asm volatile("" : "+v"(k[0]), "+v"(k[1]), "+v"(k[2]), "+v"(k[3])::"memory");
+      if (st + 1 < nst)
+        request(base, st + 1);
+      else if (base + NT < n)
+        request(base + NT, 0);
+#define ELM_SCORE_STEP(m) acc[(m) & 3] = acc[(m) & 3] + row_bcast<m>(qr) * k[(m) >> 2][(m) & 3];
+#define ELM_SCORE_STEP4(u) ELM_SCORE_STEP(4 * (u)) ELM_SCORE_STEP(4 * (u) + 1) ELM_SCORE_STEP(4 * (u) + 2) ELM_SCORE_STEP(4 * (u) + 3)
+      const int nd4 = min(4, hd4 - 4 * st);
+      ELM_SCORE_STEP4(0)
+      if (nd4 > 1) { ELM_SCORE_STEP4(1) }
+      if (nd4 > 2) { ELM_SCORE_STEP4(2) }
+      if (nd4 > 3) { ELM_SCORE_STEP4(3) }
+#undef ELM_SCORE_STEP4
+#undef ELM_SCORE_STEP
+    }
+    if (base + lane < n) {
+      const float sj = ((acc[0] + acc[1]) + (acc[2] + acc[3])) * scale;
+      sc[base + lane] = sj;
+      mx = fmaxf(mx, sj);
+    }
+  }
+  mx = wave_max(mx);
+  if (lane == 0) red[w] = mx;
+  __syncthreads();
+  mx = red[0];
+#pragma unroll
+  for (int i = 1; i < kStepWaves; ++i) mx = fmaxf(mx, red[i]);
+  const int n16 = (n + 15) & ~15;
+  for (int j = tid; j < n16; j += NT) sc[j] = j < n ? elm_expf_tab(sc[j] - mx, etab) : 0.f;
+  __syncthreads();
+
+  // waves 1, 2, ..: dim 64 (w - 1) + lane of the output
+  const int dim = 64 * (w - 1) + lane, dc = min(max(dim, 0), hd - 1);
+  const bool adds = w > 0 && 64 * (w - 1) < hd;
+  const float* const vd = vh + dc;
+  float v[4][16], vlast = 0.f;
+  auto load = [&](int j0, float (&b)[16]) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) b[u] = vd[(int64_t)min(j0 + u, rlast) * hd];
+  };
+  if (w == 0) {
+    float sum = 0.f;
+    for (int g0 = 0; g0 < n16; g0 += 256) sum = ordered_sum256(sc + g0, min(16, (n16 - g0) >> 4), sum);
+    if (lane == 0) inv_s = 1.0f / sum;
+  } else if (adds) {
+    if (FUSE) vlast = vnew[kvh * hd + dc];
+    load(0, v[0]);
+    load(16, v[1]);
+    load(32, v[2]);
+    load(48, v[3]);
+  }
+  lds_barrier();  // the values stay in flight
+  if (!adds) return;
+  const float inv = inv_s;
+  float acc = 0.f;
+#define ELM_OUT_STEP(m)                                    \
+  {                                                        \
+    const float pv = row_bcast<m>(p) * b[m];               \
+    acc = acc + (full || j0 + (m) < nc ? pv : 0.f);        \
+  }
+  auto batch = [&](int j0, const float (&b)[16], bool full) __attribute__((always_inline)) {
+    const float p = sc[j0 + (lane & 15)] * inv;
+    ELM_OUT_STEP(0) ELM_OUT_STEP(1) ELM_OUT_STEP(2) ELM_OUT_STEP(3) ELM_OUT_STEP(4) ELM_OUT_STEP(5) ELM_OUT_STEP(6)
+    ELM_OUT_STEP(7) ELM_OUT_STEP(8) ELM_OUT_STEP(9) ELM_OUT_STEP(10) ELM_OUT_STEP(11) ELM_OUT_STEP(12) ELM_OUT_STEP(13)
+    ELM_OUT_STEP(14) ELM_OUT_STEP(15)
+  };
+#undef ELM_OUT_STEP
+  int j0 = 0;
+  for (; j0 + 64 <= nc; j0 += 64) {
+    batch(j0, v[0], true);
+    load(j0 + 64, v[0]);
+    batch(j0 + 16, v[1], true);
+    load(j0 + 80, v[1]);
+    batch(j0 + 32, v[2], true);
+    load(j0 + 96, v[2]);
+    batch(j0 + 48, v[3], true);
+    load(j0 + 112, v[3]);
+  }
+  if (j0 < nc) batch(j0, v[0], false);
+  if (j0 + 16 < nc) batch(j0 + 16, v[1], false);
+  if (j0 + 32 < nc) batch(j0 + 32, v[2], false);
+  if (j0 + 48 < nc) batch(j0 + 48, v[3], false);
+  if (FUSE) acc = acc + (sc[nc] * inv) * vlast;  // the step's own value
+  if (dim < hd) out[(int64_t)t * qd + h * hd + dim] = acc;
+}
+
 // ---------------------------------------------------------------- EMBED
 
 // y[t][k] = dequantize_row(table, tokens[t])[k] read from the repacked weight layout:
@@ -1423,12 +1836,39 @@ size_t attention_global_score_bytes(int T, int pos0, bool pos_dev, int n_heads, 
   return (size_t)T * n_heads * (size_t)((n_cap + 63) & ~63) * sizeof(float);
 }
 
+// attention_rows_kernel for R rows per workgroup: the score row stride (a multiple of 4 that spreads the rows over the LDS
+// banks) and the LDS it takes
+static int attn_rows_stride(int n_cap) { return ((n_cap + 63) & ~63) + 20; }
+static size_t attention_rows_lds_bytes(int R, int hd, int n_cap) {
+  return ((size_t)R * attn_rows_stride(n_cap) + 256 + 4 * 1024 + (size_t)R * ((hd + 15) & ~15)) * sizeof(float);
+}
+template <int R>
+static hipError_t launch_attention_rows(const float* q, float* out, const float* kc, const float* vc, int T, int pos0, int grp,
+                                        int n_kv, int hd, int max_ctx, const float* rcos, const float* rsin, int8_t* xq,
+                                        float* xd, int Tpad, hipStream_t s) {
+  const dim3 grid(n_kv, (T * grp + R - 1) / R);
+  const size_t lds = attention_rows_lds_bytes(R, hd, pos0 + T);
+  const int scs = attn_rows_stride(pos0 + T);
+  if (hd <= 64)
+    attention_rows_kernel<R, 2><<<grid, 256, lds, s>>>(q, out, kc, vc, pos0, T, grp, n_kv, hd, max_ctx, scs, rcos, rsin, xq, xd, Tpad);
+  else
+    attention_rows_kernel<R, 1><<<grid, 256, lds, s>>>(q, out, kc, vc, pos0, T, grp, n_kv, hd, max_ctx, scs, rcos, rsin, xq, xd, Tpad);
+  return hipGetLastError();
+}
+
+static size_t attention_step_lds_bytes(int hd, int n_cap) {
+  return ((size_t)((n_cap + 15) & ~15) + 256 + kStepWaves * 1024 + 2 * (size_t)((hd + 15) & ~15)) * sizeof(float);
+}
+
 // the attention kernels keep a whole score row (and a chunk of values) in LDS: allow them up to kMaxAttnLds
 bool raise_lds_limit() {
   const void* kernels[] = {(const void*)attention_kernel<64, false>, (const void*)attention_kernel<0, false>,
                            (const void*)attention_kernel<64, true>, (const void*)attention_kernel<0, true>,
                            (const void*)attention_prefill_kernel, (const void*)attention_decode64_kernel,
-                           (const void*)attention_prefill64_kernel};
+                           (const void*)attention_prefill64_kernel,
+                           (const void*)attention_step_kernel<true>, (const void*)attention_step_kernel<false>,
+                           (const void*)attention_rows_kernel<8, 1>, (const void*)attention_rows_kernel<8, 2>,
+                           (const void*)attention_rows_kernel<4, 1>, (const void*)attention_rows_kernel<4, 2>};
   for (const void* k : kernels) {
     hipFuncAttributes fa;
     if (hipFuncGetAttributes(&fa, k) != hipSuccess || fa.sharedSizeBytes + kMaxAttnLds > kMaxLds) return false;
@@ -1447,9 +1887,28 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, floa
   // one token, and chunks on the head-size-64 prefill kernel: the append runs inside the attention
   // kernel; other chunks append every key first
   const bool fuse = T == 1;
+  const int grp = n_heads / n_kv;
+  const bool quant = xq && xd && quantized;
   const size_t lds_pf = ((size_t)kAttnQ * hd + (size_t)kAttnQ * ((n_cap + 63) & ~63) + (size_t)kAttnPVPos * hd) * 4;
   const size_t lds_pf64 = ((size_t)2 * kPfRows * 64 + (size_t)kAttnQ * ((n_cap + 255) & ~255) + (size_t)kAttnQ * 64) * 4;
-  const bool pf64 = !fuse && hd == 64 && lds_pf64 <= kMaxAttnLds && !pos_dev;
+  // A chunk of at most one (token, head) per CU: a 1024-thread workgroup each (32 heads of size 128 over 1000 cached
+  // positions: 35 / 38 us for 2 / 8 tokens, against 51 us with rows of four in 256-thread workgroups; 16 tokens 55 against
+  // 52). At head size 64 only where no GEMM operand is asked for (8 tokens of 9 heads over 300 positions: 13.7 against 17.9
+  // us with attention_prefill64_kernel). One token: always, but for the head-size-64 kernel's caches (it takes the step's
+  // rows before it knows the position: 6.0 against 8.6 us at 200 positions, 15.4 against 19.9 at 700).
+  const bool step_fits = attention_step_lds_bytes(hd, n_cap) <= kMaxAttnLds;
+  const bool step = step_fits && (fuse ? hd != 64 || attention_decode_lds_bytes(n_cap) > kMaxAttnLds
+                                       : !pos_dev && (int64_t)T * n_heads <= 256 && (hd != 64 || !quant));
+  // Longer chunks: attention_rows_kernel, at head size 64 from 4096 (token, head) pairs on (9 heads: 512 tokens 31 against
+  // 48 us with attention_prefill64_kernel, 128 tokens 11 against 8.4; 32 heads, 64 tokens at 600 positions 34 against 32).
+  // R = 8 rows a workgroup read the keys half as often as 4; 4 fill the chip at fewer rows and keep more workgroups per CU
+  // where the score rows are long (32 heads of size 128: 256 tokens at 256 positions 80 against 86 us; 128 tokens 19.5
+  // against 17.4; 512 at 1500 986 against 613).
+  auto wgs = [&](int R) { return (int64_t)n_kv * (((int64_t)T * grp + R - 1) / R); };
+  const int R = wgs(8) >= 1024 && 3 * attention_rows_lds_bytes(8, hd, n_cap) <= kMaxLds ? 8 : 4;
+  const bool rows = !fuse && !pos_dev && !step && wgs(R) / n_kv < 65536 && (hd != 64 || (int64_t)T * n_heads >= 4096) &&
+                    attention_rows_lds_bytes(R, hd, n_cap) <= kMaxAttnLds;
+  const bool pf64 = !fuse && hd == 64 && lds_pf64 <= kMaxAttnLds && !pos_dev && !step && !rows;
   if (!fuse && !pf64) {
     kv_append_kernel<<<T * n_kv, 64, 0, s>>>(k, v, kc, vc, pos0, pos_dev, n_kv, hd, max_ctx, rcos, rsin);
     hipError_t e = hipGetLastError();
@@ -1459,9 +1918,25 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, floa
   const float* vn = fuse ? v : nullptr;
   static const bool lds_ok = raise_lds_limit();  // once per process (the attribute holds for the kernel)
   if (!lds_ok) return hipErrorInvalidValue;
+  if (step) {
+    const dim3 grid(n_kv, grp, T);
+    const size_t lds = attention_step_lds_bytes(hd, n_cap);
+    if (fuse)
+      attention_step_kernel<true><<<grid, 64 * kStepWaves, lds, s>>>(q, out, kc, vc, pos0, pos_dev, grp, n_kv, hd, max_ctx,
+                                                                     n_cap, rcos, rsin, k, v);
+    else
+      attention_step_kernel<false><<<grid, 64 * kStepWaves, lds, s>>>(q, out, kc, vc, pos0, nullptr, grp, n_kv, hd, max_ctx,
+                                                                      n_cap, rcos, rsin, nullptr, nullptr);
+    return hipGetLastError();
+  }
+  if (rows) {
+    const hipError_t e = R == 8 ? launch_attention_rows<8>(q, out, kc, vc, T, pos0, grp, n_kv, hd, max_ctx, rcos, rsin, quant ? xq : nullptr, xd, Tpad, s)
+                                : launch_attention_rows<4>(q, out, kc, vc, T, pos0, grp, n_kv, hd, max_ctx, rcos, rsin, quant ? xq : nullptr, xd, Tpad, s);
+    if (e == hipSuccess && quant) *quantized = true;
+    return e;
+  }
   if (pf64) {
     const int ngr = (T + kAttnQ - 1) / kAttnQ;
-    const bool quant = xq && xd && quantized;
     attention_prefill64_kernel<<<dim3(ngr, n_heads / n_kv, n_kv), 256, lds_pf64, s>>>(
         q, out, kc, vc, pos0, T, n_heads / n_kv, n_kv, max_ctx, n_cap, rcos, rsin, quant ? xq : nullptr,
         quant ? xd : nullptr, Tpad, k, v);
@@ -1471,7 +1946,6 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, floa
   }
   if (!fuse && hd == 64 && lds_pf <= kMaxAttnLds) {
     const int ngr = (T + kAttnQ - 1) / kAttnQ;
-    const bool quant = xq && xd && quantized;
     attention_prefill_kernel<<<n_heads * ngr, 256, lds_pf, s>>>(q, out, kc, vc, pos0, T, n_heads, n_kv, max_ctx, n_cap,
                                                                 rcos, rsin, quant ? xq : nullptr,
                                                                 quant ? xd : nullptr, Tpad);
