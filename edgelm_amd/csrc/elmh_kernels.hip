@@ -20,6 +20,7 @@
 #include "elm_sum.h"
 
 #include <cstring>
+#include <type_traits>
 
 namespace elmh {
 namespace {
@@ -2118,6 +2119,8 @@ done:
 
 // ---------------------------------------------------------------- f32-activation paths
 
+typedef float v4fl __attribute__((ext_vector_type(4)));
+
 // The target owning tile `tile` of an f32-activation launch (tile made relative to it): the target
 // count and the tile starts, pinned in scalar registers, come with the kernel's other arguments in
 // one batch of scalar loads; the target's fields then take one more (uniform) load through the
@@ -2468,16 +2471,7 @@ __global__ __launch_bounds__(64) void gemv_f32act_q8_kernel(const F32Args a) {
 
 // T > 1 (kernels_cpu.cpp:369-371, 401-403): the weight tile is dequantized (float(q) * s, one
 // rounding) and dotted in dot_f32_scalar's four chains (chain c takes i = c mod 4 in order, the
-// K mod 4 tail goes to chain 0); y = (res or 0) + dot. The chains are independent, so four lanes
-// take one (row, kF32TT tokens) tile, a chain each: a workgroup is 64 rows x kF32TT tokens (2
-// tokens measured faster than 4 or 8 at the 135M model's 128-token prefill, which has too few
-// (row, token) pairs to fill the chip with more tokens per lane). x is staged
-// through LDS by chain ([token][chain][k / 4], so a lane reads four of its chain's values at
-// once), and the row's four lanes read the same 16 weight bytes, each using its own four.
-constexpr int kF32TT = 2;
-constexpr int kF32Chunk = 2048;
-constexpr int kF32ChainStride = kF32Chunk / 4 + 4;  // floats; the +4 spreads the staging writes over banks
-
+// K mod 4 tail goes to chain 0); y = (res or 0) + dot.
 template <int WDT>
 __device__ __forceinline__ float deq1(const uint8_t* __restrict__ data, const float* __restrict__ scales,
                                       int64_t nbase, int H, int i, int n) {
@@ -2489,132 +2483,173 @@ __device__ __forceinline__ float deq1(const uint8_t* __restrict__ data, const fl
   return (float)((int)(e >= 16 ? byte >> 4 : byte & 0x0F) - 8) * scales[item];
 }
 
-// The 16 weight bytes that hold elements i .. i + 15 of row n (i % 16 == 0) and their scale
-struct WChunk {
-  uint4 q;
-  float s;
-};
-template <int WDT>
-__device__ __forceinline__ WChunk load_chunk(const uint8_t* __restrict__ data, const float* __restrict__ scales,
-                                             int64_t nbase, int H, int i, int n) {
-  const int64_t item = nbase + (int64_t)(i >> 5) * H;
-  if (WDT == WQ8) return {*reinterpret_cast<const uint4*>(data + item * 32 + (i & 31)), scales[n]};
-  return {*reinterpret_cast<const uint4*>(data + item * 16), scales[item]};  // the group: byte m holds m, m + 16
-}
-// chain c's four dequantized weights of the chunk: elements i + c + 4m, m = 0 .. 3
-template <int WDT>
-__device__ __forceinline__ float4 chunk_chain(const WChunk& w, int i, int c) {
-  float4 r;
-  if (WDT == WQ8) {
-    r.x = (float)(int8_t)((w.q.x >> (8 * c)) & 0xFF) * w.s;
-    r.y = (float)(int8_t)((w.q.y >> (8 * c)) & 0xFF) * w.s;
-    r.z = (float)(int8_t)((w.q.z >> (8 * c)) & 0xFF) * w.s;
-    r.w = (float)(int8_t)((w.q.w >> (8 * c)) & 0xFF) * w.s;
-  } else {
-    const int sh = 8 * c + ((i & 31) >= 16 ? 4 : 0);
-    r.x = (float)((int)((w.q.x >> sh) & 0x0F) - 8) * w.s;
-    r.y = (float)((int)((w.q.y >> sh) & 0x0F) - 8) * w.s;
-    r.z = (float)((int)((w.q.z >> sh) & 0x0F) - 8) * w.s;
-    r.w = (float)((int)((w.q.w >> sh) & 0x0F) - 8) * w.s;
-  }
-  return r;
-}
-constexpr int kF32Ahead = 4;  // 16-element steps whose weights are in flight
-
-template <int WDT, bool SW>
-__global__ __launch_bounds__(256) void gemm_f32act_kernel(const F32Args a) {
-  __shared__ __align__(16) float sxp[kF32TT][4][kF32ChainStride];
-  int grp = blockIdx.y;
+// The chains are independent, so they run from a tile in LDS: a workgroup is 16 RY rows x 8 TX tokens. Lane 4 m + c of a wave runs chain c of
+// rows m, m + 16, .. for the wave's TX tokens (gate and up with SW), so that a quad's four lanes hold one (row, token)'s
+// four chains. 16 P k's per step are staged in two buffers with one barrier per step: the weights dequantized once for the
+// workgroup, both operands as 16-byte slots of one chain's next four values (k = 16 h + 4 u + c, u = 0 .. 3), [h][item][c],
+// which lanes read and write without bank conflicts; the global loads run two steps ahead, in registers. The vector ALU
+// (4.3 clocks per 64 multiplies and adds of a wave at two waves per SIMD: they may not be fused) and the LDS reads (RY + TX
+// slots for RY TX multiplies and adds of four, 8 clocks each) bound it where the tile is large, the barrier and the latencies
+// behind it at each step where it is small (P = 8 against 4 at 4096 x 4096 q4: 24 against 37 us for 2 tokens, 65 against 68 for
+// 64; 16 pieces went to scratch). Against one workgroup per 64 rows and 2 tokens, which dequantized every weight again for each
+// pair of tokens: 2 tokens 50 -> 24 us, 16 69 -> 29, 64 134 -> 65, 256 461 -> 189; a form with a lane per row and the x values
+// broadcast by the multiply (row_bcast, 6.1 clocks) took 38, 52, 81 and 244 us.
+constexpr int kF32TWaves = 8;
+template <int WDT, bool SW, int RY, int TX, int P>
+__global__ __launch_bounds__(64 * kF32TWaves) void gemm_f32act_tile_kernel(const F32Args a) {
+  constexpr int NSEL = SW ? 2 : 1, NT = 64 * kF32TWaves, R = 16 * RY, TT = kF32TWaves * TX;
+  constexpr int WSL = 4 * P * R, XSL = 4 * P * TT;  // slots of a step (P 16-k pieces) per selection, and of x
+  constexpr int NW = (WSL + NT - 1) / NT, NX = (XSL + NT - 1) / NT;
+  __shared__ __align__(16) v4fl wl[2][NSEL][P][R * 4], xl[2][P][TT * 4];
+  const int tt = a.rt;  // token tiles: consecutive workgroups share their weight rows
+  int grp = blockIdx.x / tt;
+  const int t0 = (blockIdx.x - grp * tt) * TT;
   const GemvTarget tg = f32_target<SW>(a, grp);
   const int K = a.K, K4 = K & ~3, H = a.H, nb = a.nb, T = a.T;
-  const int t0 = blockIdx.x * kF32TT, c = threadIdx.x & 3;
-  const int n = grp * 64 + (threadIdx.x >> 2);  // rows past N: padding (rows_pad % 64 == 0)
-  const int64_t nbase = (int64_t)(n / H) * nb * H + (n % H);
-  float s[kF32TT], su[kF32TT];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = grp * R;
+  const int nch = (K4 + 15) >> 4, nst = (nch + P - 1) / P;  // 16-k pieces, and steps of P
+  // staging tasks: slot j = tid + NT i of a selection's weights (piece j / (4 R), row j / 4 % R, chain j % 4), and of x
+  v4u wq[2][NSEL][NW];
+  float ws[2][NSEL][NW];
+  float xq[2][NX][4];
+  auto fetch = [&](int st, v4u (&q)[NSEL][NW], float (&sc)[NSEL][NW], float (&x)[NX][4]) {
 #pragma unroll
-  for (int t = 0; t < kF32TT; ++t) s[t] = su[t] = 0.f;
-  for (int k0 = 0; k0 < K4; k0 += kF32Chunk) {
-    const int klen = min(kF32Chunk, K4 - k0);
-    __syncthreads();
-    for (int i = threadIdx.x; i < kF32TT * kF32Chunk; i += 256) {
-      const int t = i / kF32Chunk, k = i - t * kF32Chunk;
-      if (k < klen) sxp[t][k & 3][k >> 2] = t0 + t < T ? a.x[(int64_t)(t0 + t) * K + k0 + k] : 0.f;
+    for (int i = 0; i < NW; ++i) {
+      const int j = tid + NT * i, h = P * st + j / (4 * R), n = n0 + (j >> 2) % R;  // rows past N: padding
+      const int64_t item = (int64_t)(n / H) * nb * H + (n % H) + (int64_t)min(h >> 1, nb - 1) * H;
+      if (WSL % NT == 0 || j < WSL)
+#pragma unroll
+        for (int s = 0; s < NSEL; ++s) {
+          const uint8_t* const data = SW && s ? a.tg[1].data : tg.data;
+          q[s][i] = *reinterpret_cast<const v4u*>(WDT == WQ8 ? data + item * 32 + 16 * (h & 1) : data + item * 16);
+          sc[s][i] = (SW && s ? a.tg[1].scales : tg.scales)[WDT == WQ8 ? n : item];
+        }
     }
-    __syncthreads();
-    // the chunk's 16-element steps; each step's weights are loaded kF32Ahead steps before it
-    const int nst = klen >> 4;
-    WChunk wr[kF32Ahead], ur[kF32Ahead];
 #pragma unroll
-    for (int u = 0; u < kF32Ahead; ++u)
-      if (u < nst) {
-        wr[u] = load_chunk<WDT>(tg.data, tg.scales, nbase, H, k0 + 16 * u, n);
-        if (SW) ur[u] = load_chunk<WDT>(a.tg[1].data, a.tg[1].scales, nbase, H, k0 + 16 * u, n);
+    for (int i = 0; i < NX; ++i) {
+      const int j = tid + NT * i, h = P * st + j / (4 * TT), t = t0 + (j >> 2) % TT;
+      if (XSL % NT == 0 || j < XSL) {
+        const float* const xr = a.x + (int64_t)min(t, T - 1) * K + (j & 3);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[i][u] = xr[min(16 * h + 4 * u, K4 - 4)];  // past the end: any value of the row
       }
-    for (int s0 = 0; s0 < nst; s0 += kF32Ahead) {
+    }
+  };
+  auto stage = [&](int st, int buf, const v4u (&q)[NSEL][NW], const float (&sc)[NSEL][NW], const float (&x)[NX][4]) {
 #pragma unroll
-      for (int u = 0; u < kF32Ahead; ++u) {
-        const int st = s0 + u, ii = k0 + 16 * st;
-        if (st < nst) {
-          const float4 w = chunk_chain<WDT>(wr[u], ii, c);
-          const float4 wu = SW ? chunk_chain<WDT>(ur[u], ii, c) : w;
-          if (st + kF32Ahead < nst) {
-            wr[u] = load_chunk<WDT>(tg.data, tg.scales, nbase, H, ii + 16 * kF32Ahead, n);
-            if (SW) ur[u] = load_chunk<WDT>(a.tg[1].data, a.tg[1].scales, nbase, H, ii + 16 * kF32Ahead, n);
-          }
+    for (int i = 0; i < NW; ++i) {
+      const int j = tid + NT * i, hp = j / (4 * R), h = P * st + hp, c8 = 8 * (j & 3);
+      if (WSL % NT == 0 || j < WSL)
 #pragma unroll
-          for (int t = 0; t < kF32TT; ++t) {
-            const float4 xv = *reinterpret_cast<const float4*>(&sxp[t][c][(ii - k0) >> 2]);
-            s[t] = s[t] + xv.x * w.x;
-            s[t] = s[t] + xv.y * w.y;
-            s[t] = s[t] + xv.z * w.z;
-            s[t] = s[t] + xv.w * w.w;
-            if (SW) {
-              su[t] = su[t] + xv.x * wu.x;
-              su[t] = su[t] + xv.y * wu.y;
-              su[t] = su[t] + xv.z * wu.z;
-              su[t] = su[t] + xv.w * wu.w;
-            }
+        for (int s = 0; s < NSEL; ++s) {
+          v4fl v;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if (WDT == WQ8)
+              v[u] = (float)(int8_t)((q[s][i][u] >> c8) & 0xFF) * sc[s][i];
+            else  // byte m of the group holds elements m and m + 16
+              v[u] = ((float)((q[s][i][u] >> (c8 + 4 * (h & 1))) & 0x0Fu) - 8.f) * sc[s][i];
           }
+          if (16 * h + 16 > K4)  // the row's last piece: zeros past its last whole four (adding them changes no sum)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = 16 * h + 4 * u < K4 ? v[u] : 0.f;
+          wl[buf][s][hp][j % (4 * R)] = v;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int j = tid + NT * i, hp = j / (4 * TT), h = P * st + hp;
+      if (XSL % NT == 0 || j < XSL) {
+        v4fl v = {x[i][0], x[i][1], x[i][2], x[i][3]};
+        if (16 * h + 16 > K4)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] = 16 * h + 4 * u < K4 ? v[u] : 0.f;
+        xl[buf][hp][j % (4 * TT)] = v;
+      }
+    }
+  };
+  float acc[NSEL][RY][TX];
+#pragma unroll
+  for (int s = 0; s < NSEL; ++s)
+#pragma unroll
+    for (int r = 0; r < RY; ++r)
+#pragma unroll
+      for (int t = 0; t < TX; ++t) acc[s][r][t] = 0.f;
+  const bool live = t0 + w * TX < T;  // waves past the last token only stage
+  auto step = [&](int st, int buf) __attribute__((always_inline)) {
+    const int np = min(P, nch - P * st);  // P but in the last step
+    v4fl wv[2][NSEL][RY], xv[2][TX];
+    auto read = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < NSEL; ++s)
+#pragma unroll
+        for (int r = 0; r < RY; ++r) wv[h & 1][s][r] = wl[buf][s][h][64 * r + lane];
+#pragma unroll
+      for (int t = 0; t < TX; ++t) xv[h & 1][t] = xl[buf][h][4 * (w * TX + t) + (lane & 3)];
+    };
+    read(0);
+#pragma unroll
+    for (int h = 0; h < P; ++h) {
+      if (h >= np) break;
+      if (h + 1 < P) read(h + 1);  // the next piece (in the last step perhaps an old one, unused) before this one's multiplies
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int s = 0; s < NSEL; ++s)
+#pragma unroll
+          for (int r = 0; r < RY; ++r)
+#pragma unroll
+            for (int t = 0; t < TX; ++t) acc[s][r][t] = acc[s][r][t] + xv[h & 1][t][u] * wv[h & 1][s][r][u];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (nst > 0) {  // K >= 4
+    fetch(0, wq[0], ws[0], xq[0]);
+    fetch(1, wq[1], ws[1], xq[1]);
+    stage(0, 0, wq[0], ws[0], xq[0]);
+  }
+  for (int st = 0; st < nst; st += 2) {
+    lds_barrier();  // step st is in buffer 0, and every wave has finished step st - 1 (buffer 1)
+    fetch(st + 2, wq[0], ws[0], xq[0]);
+    stage(st + 1, 1, wq[1], ws[1], xq[1]);
+    if (live) step(st, 0);
+    if (st + 1 >= nst) break;
+    lds_barrier();
+    fetch(st + 3, wq[1], ws[1], xq[1]);
+    stage(st + 2, 0, wq[0], ws[0], xq[0]);
+    if (live) step(st + 1, 1);
+  }
+  if (!live) return;
+  const int c = lane & 3;
+#pragma unroll
+  for (int r = 0; r < RY; ++r) {
+    const int n = n0 + 16 * r + (lane >> 2);
+    const int64_t nbase = (int64_t)(n / H) * nb * H + (n % H);
+#pragma unroll
+    for (int t = 0; t < TX; ++t) {
+      const int tk = t0 + w * TX + t;
+      float dot[NSEL];
+#pragma unroll
+      for (int s = 0; s < NSEL; ++s) {
+        float v = acc[s][r][t];
+        if (c == 0 && tk < T)
+          for (int i = K4; i < K; ++i)  // tail (K % 4) into the first chain
+            v = v + a.x[(int64_t)tk * K + i] * deq1<WDT>(SW && s ? a.tg[1].data : tg.data, SW && s ? a.tg[1].scales : tg.scales, nbase, H, i, n);
+        const float p = v + dpp_f<kDppQuadXor1>(v);  // lane 0: s0 + s1, lane 2: s2 + s3
+        dot[s] = p + dpp_f<kDppQuadXor2>(p);
+      }
+      if (c == 0 && n < tg.N && tk < T) {
+        const int64_t o = (int64_t)tk * tg.N + n;
+        if (SW) {
+          const float g = 0.f + dot[0], u = 0.f + dot[NSEL - 1];
+          tg.y[o] = silu_exact(g) * u;
+        } else {
+          tg.y[o] = (tg.res ? tg.res[o] : 0.f) + dot[0];
         }
       }
     }
-    int i = k0 + 16 * nst;
-    for (; i < k0 + klen; i += 4) {  // the last chunk's steps past its last 16-element run
-      const float w = deq1<WDT>(tg.data, tg.scales, nbase, H, i + c, n);
-      const float wu = SW ? deq1<WDT>(a.tg[1].data, a.tg[1].scales, nbase, H, i + c, n) : w;
-#pragma unroll
-      for (int t = 0; t < kF32TT; ++t) {
-        const float xv = sxp[t][c][(i - k0) >> 2];
-        s[t] = s[t] + xv * w;
-        if (SW) su[t] = su[t] + xv * wu;
-      }
-    }
-  }
-  if (c == 0)
-    for (int i = K4; i < K; ++i) {  // tail (K % 4) into the first chain
-      const float w = deq1<WDT>(tg.data, tg.scales, nbase, H, i, n);
-      const float wu = SW ? deq1<WDT>(a.tg[1].data, a.tg[1].scales, nbase, H, i, n) : w;
-#pragma unroll
-      for (int t = 0; t < kF32TT; ++t) {
-        const float xv = t0 + t < T ? a.x[(int64_t)(t0 + t) * K + i] : 0.f;
-        s[t] = s[t] + xv * w;
-        if (SW) su[t] = su[t] + xv * wu;
-      }
-    }
-#pragma unroll
-  for (int t = 0; t < kF32TT; ++t) {
-    const float p = s[t] + __shfl_xor(s[t], 1);  // lane 0: s0 + s1, lane 2: s2 + s3
-    const float dot = p + __shfl_xor(p, 2);
-    float out;
-    if (SW) {
-      const float pu = su[t] + __shfl_xor(su[t], 1);
-      const float g = 0.f + dot;
-      const float u = 0.f + (pu + __shfl_xor(pu, 2));
-      out = silu_exact(g) * u;
-    } else {
-      out = (t0 + t < T && tg.res ? tg.res[(int64_t)(t0 + t) * tg.N + n] : 0.f) + dot;
-    }
-    if (c == 0 && n < tg.N && t0 + t < T) tg.y[(int64_t)(t0 + t) * tg.N + n] = out;
   }
 }
 
@@ -3090,23 +3125,46 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
       gemv_f32act_q8_kernel<false><<<groups, 64, lds, s>>>(b);
     }
   } else {
-    // grid x: kF32TT-token tiles (consecutive workgroups share their weight rows), y: 64-row groups
-    F32Args b = a;
-    int groups = 0;
-    for (int i = 0; i < n; ++i) {
-      b.tile_start[i] = groups;
-      groups += (a.tg[i].N + 63) / 64;
-    }
-    b.tile_start[n] = groups;
-    if (groups < 1 || groups > 65535) return hipErrorInvalidValue;
-    const dim3 grid((a.T + kF32TT - 1) / kF32TT, groups);
-    if (dtype == WQ8) {
-      if (swiglu) gemm_f32act_kernel<WQ8, true><<<grid, 256, 0, s>>>(b);
-      else gemm_f32act_kernel<WQ8, false><<<grid, 256, 0, s>>>(b);
-    } else {
-      if (swiglu) gemm_f32act_kernel<WQ4, true><<<grid, 256, 0, s>>>(b);
-      else gemm_f32act_kernel<WQ4, false><<<grid, 256, 0, s>>>(b);
-    }
+    // The largest tile that makes at least two workgroups per CU (one for 32 rows x 16 tokens), else 16 rows x 8 tokens: at
+    // 4096 x 4096 q4 and 256 / 128 / 64 / 32 / 16 tokens 64 x 32 tiles take 189 / 114 / 109 / 105 / 95 us, 64 x 16 220 / 115 /
+    // 71 / 68 / 67, 32 x 16 240 / 124 / 65 / 41 / 40, 16 x 8 343 / 179 / 95 / 50 / 29. SwiGLU holds both selections, so at most
+    // 32 x 16 (3648 x 1088, 175 tokens, with its down projection: 148 us, 185 with 64 x 16).
+    auto wgs = [&](int ry, int tx) {
+      int64_t g = 0;
+      for (int i = 0; i < n; ++i) g += (a.tg[i].N + 16 * ry - 1) / (16 * ry);
+      return g * ((a.T + kF32TWaves * tx - 1) / (kF32TWaves * tx));
+    };
+    const int64_t big = 512, mid = 256;
+    auto go = [&](auto ry, auto tx, auto pp) {
+      constexpr int RY = decltype(ry)::value, TX = decltype(tx)::value, P = decltype(pp)::value;
+      F32Args b = a;
+      int groups = 0;
+      for (int i = 0; i < n; ++i) {
+        b.tile_start[i] = groups;
+        groups += (a.tg[i].N + 16 * RY - 1) / (16 * RY);
+      }
+      b.tile_start[n] = groups;
+      b.rt = (a.T + kF32TWaves * TX - 1) / (kF32TWaves * TX);
+      if (groups < 1 || (int64_t)groups * b.rt > INT32_MAX) return hipErrorInvalidValue;
+      const int grid = groups * b.rt, threads = 64 * kF32TWaves;
+      if constexpr (RY <= 2) {
+        if (swiglu) {
+          if (dtype == WQ8) gemm_f32act_tile_kernel<WQ8, true, RY, TX, P><<<grid, threads, 0, s>>>(b);
+          else gemm_f32act_tile_kernel<WQ4, true, RY, TX, P><<<grid, threads, 0, s>>>(b);
+          return hipGetLastError();
+        }
+      }
+      if (dtype == WQ8) gemm_f32act_tile_kernel<WQ8, false, RY, TX, P><<<grid, threads, 0, s>>>(b);
+      else gemm_f32act_tile_kernel<WQ4, false, RY, TX, P><<<grid, threads, 0, s>>>(b);
+      return hipGetLastError();
+    };
+    using std::integral_constant;
+    if (!swiglu && wgs(4, 4) >= big)
+      return go(integral_constant<int, 4>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{});
+    if (!swiglu && wgs(4, 2) >= big)
+      return go(integral_constant<int, 4>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+    if (wgs(2, 2) >= mid) return go(integral_constant<int, 2>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+    return go(integral_constant<int, 1>{}, integral_constant<int, 1>{}, integral_constant<int, 8>{});
   }
   return hipGetLastError();
 }

@@ -1,0 +1,54 @@
+"""The f32-activation kernels at the sizes where their dispatch or tiles turn, bit for bit against the oracle: the LDS-tile
+GEMM's four tiles with ragged rows, tokens and row lengths (K past and short of whole 16s, 32s and 128s, K below 4), several
+targets."""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import bits_equal
+from edgelm_amd import elmh as E
+
+pytestmark = pytest.mark.gpu
+
+
+def up(ctx, w):
+    return ctx.upload(w.dtype, w.rows, w.cols, w.data, w.scales)
+
+
+def weight(r, n, k, dt):
+    return O.make_weight(r.normal(0, 0.05, (n, k)).astype(np.float32), dt)
+
+
+# (rows, K, T): 64 x 32 tiles (512 workgroups), 64 x 16, 32 x 16, 16 x 8
+TILES = [(2000, 96, 505), (1030, 160, 490), (1000, 288, 126), (70, 544, 9), (33, 2080, 2), (17, 32, 3)]
+
+
+@pytest.mark.parametrize("shape", TILES, ids=["x".join(map(str, s)) for s in TILES])
+@pytest.mark.parametrize("dt", [O.Q8, O.Q4])
+def test_f32act_gemm_tiles(ctx, dt, shape):
+    n, k, T = shape
+    r = np.random.default_rng(n + k)
+    for kk in [k] + ([k - 1, k - 18, k - 30] if dt == O.Q8 else []):
+        ws = [weight(r, n, kk, dt), weight(r, 40, kk, dt)]
+        x = r.normal(0, 1, (T, kk)).astype(np.float32)
+        res = r.normal(0, 1, (T, n)).astype(np.float32)
+        dws = [up(ctx, w) for w in ws]
+        print(f"[gpu] f32act gemm tiles dt={dt} {n}x{kk} T={T}", flush=True)
+        got = ctx.matmul(x, dws, [res, None], act=E.ACT_F32)
+        for g, w in zip(got, O.cpu_matmul(x, ws, [res, None], act_quant=False)):
+            assert bits_equal(g, w), f"K={kk}"
+        wu = weight(r, n, kk, dt)
+        du = up(ctx, wu)
+        assert bits_equal(ctx.swiglu(x, dws[0], du, act=E.ACT_F32), O.cpu_swiglu(x, ws[0], wu, act_quant=False)), f"swiglu K={kk}"
+        for d in dws + [du]:
+            d.free()
+
+
+def test_f32act_gemm_rows_shorter_than_a_chain(ctx):
+    r = np.random.default_rng(3)
+    for k in (1, 2, 3, 4, 5, 7):
+        w = weight(r, 20, k, O.Q8)
+        x = r.normal(0, 1, (5, k)).astype(np.float32)
+        d = up(ctx, w)
+        assert bits_equal(ctx.matmul(x, [d], None, act=E.ACT_F32)[0], O.cpu_matmul(x, [w], None, act_quant=False)[0]), f"K={k}"
+        d.free()
