@@ -2246,6 +2246,123 @@ __global__ __launch_bounds__(256) void gemv_f32act_q4_kernel(const F32Args a) {
   }
 }
 
+// The same for long rows (64 < nb <= 512 groups): a thread keeps its group's 32 x values in registers and takes the group's
+// items of 8 consecutive rows (128 contiguous bytes; of gate and of up with SW), all requested at the start, so that a
+// workgroup (nb threads, or S * nb where several fit 256) reads x once for 8 S rows and not once per 1 or 2. x is requested
+// before the weights: RMSNORM's sums run while those are in flight, once per workgroup: the launch makes about two
+// workgroups per CU, which go through their tiles with the next one's weights in flight during the fold (one tile per
+// workgroup: 36 against 30 us for gate and up with RMSNORM inside). The ordered sums at both ends (RMSNORM's 1024 adds, the
+// fold) are what is left above the memory time: gate and up 2 x 14336 x 4096 55 -> 30 us, down 4096 x 14336 47 -> 16 us
+// (73 and 37 MB of weights).
+constexpr int kF32QRows = 8;
+typedef float v4flu __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned is enough
+inline bool f32q4_wide_ok(int nb, int H) { return nb > 64 && nb <= 512 && H >= kF32QRows && H % kF32QRows == 0; }
+inline int f32q4_wide_sets(int nb) { return nb <= 256 ? 256 / nb : 1; }
+template <bool SW>
+__global__ __launch_bounds__(512) void gemv_f32act_q4_wide_kernel(const F32Args a) {
+  extern __shared__ __align__(16) float f32q4w_lds[];
+  __shared__ float inv_s;
+  constexpr int NSEL = SW ? 2 : 1, RC = kF32QRows;
+  const int K = a.K, nb = a.nb, H = a.H, S = a.rt, pst = fold_stride(nb), total = a.tile_start[a.n_targets];
+  float* const P = f32q4w_lds;  // [NSEL][S * RC][pst]
+  const int tid = threadIdx.x, rs = min(tid / nb, S - 1), b = min(tid - rs * nb, nb - 1);  // spare threads repeat the last group
+  v4fl x[8], nw[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) x[u] = reinterpret_cast<const v4flu*>(a.x + 32 * b)[u];
+  if (a.nw)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) nw[u] = reinterpret_cast<const v4flu*>(a.nw + 32 * b)[u];
+  v4u wq[NSEL][RC];
+  v4fl ws[NSEL][RC / 4];
+  auto load = [&](const GemvTarget& tg, int tile) __attribute__((always_inline)) {
+    const int n0 = min(tile * S + rs, (tg.N + RC - 1) / RC - 1) * RC;  // rows past N: padding
+    const int64_t item = (int64_t)(n0 / H) * nb * H + (int64_t)b * H + n0 % H;
+#pragma unroll
+    for (int s = 0; s < NSEL; ++s) {
+      const uint8_t* const data = SW && s ? a.tg[1].data : tg.data;
+      const float* const scales = SW && s ? a.tg[1].scales : tg.scales;
+#pragma unroll
+      for (int i = 0; i < RC; ++i) wq[s][i] = reinterpret_cast<const v4u*>(data + item * 16)[i];
+#pragma unroll
+      for (int i = 0; i < RC / 4; ++i) ws[s][i] = reinterpret_cast<const v4fl*>(scales + item)[i];
+    }
+  };
+  int at = blockIdx.x, tile = at;
+  GemvTarget tg = f32_target<SW>(a, tile);
+  load(tg, tile);
+  if (a.nw) {  // as gemv_f32act_q4_kernel: squares as [accumulator][rowlen], four in-order sums
+    float* const sq = P + NSEL * S * RC * pst;
+    const int rowlen = norm_rowlen(K);
+    if (tid < nb) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const v4fl lo = {x[0][c] * x[0][c], x[1][c] * x[1][c], x[2][c] * x[2][c], x[3][c] * x[3][c]};
+        const v4fl hi = {x[4][c] * x[4][c], x[5][c] * x[5][c], x[6][c] * x[6][c], x[7][c] * x[7][c]};
+        *reinterpret_cast<v4fl*>(sq + c * rowlen + 8 * tid) = lo;
+        *reinterpret_cast<v4fl*>(sq + c * rowlen + 8 * tid + 4) = hi;
+        if (tid == nb - 1 && (nb & 1)) {  // +0.0 up to a whole batch of 16
+          *reinterpret_cast<v4fl*>(sq + c * rowlen + 8 * nb) = v4fl{0.f, 0.f, 0.f, 0.f};
+          *reinterpret_cast<v4fl*>(sq + c * rowlen + 8 * nb + 4) = v4fl{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+    }
+    lds_barrier();  // the weights stay in flight
+    if (tid < 4) {
+      const float s = ordered_sum(sq + tid * rowlen, K >> 2, 0.f);
+      const float s01 = s + dpp_f<kDppQuadXor1>(s);  // lane 0: s0 + s1, lane 2: s2 + s3
+      const float ss = s01 + dpp_f<kDppQuadXor2>(s01);
+      if (tid == 0) inv_s = 1.0f / sqrtf(ss / (float)K + a.eps);
+    }
+    lds_barrier();
+    const float inv = inv_s;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[u][c] = (x[u][c] * inv) * nw[u][c];
+  }
+  for (;;) {
+#pragma unroll
+    for (int s = 0; s < NSEL; ++s)
+#pragma unroll
+      for (int i = 0; i < RC; ++i) {
+        float g0 = 0.f, g1 = 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t lo = wq[s][i][u] & 0x0F0F0F0Fu, hi = (wq[s][i][u] >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            g0 = g0 + x[u][c] * ((float)((lo >> (8 * c)) & 0xFFu) - 8.f);
+            g1 = g1 + x[4 + u][c] * ((float)((hi >> (8 * c)) & 0xFFu) - 8.f);
+          }
+        }
+        P[(s * S * RC + rs * RC + i) * pst + b] = (g0 + g1) * ws[s][i >> 2][i & 3];
+      }
+    const GemvTarget cur = tg;
+    const int cur_tile = tile;
+    at += gridDim.x;
+    if (at < total) {  // the next tile's weights are in flight while this one is folded
+      tile = at;
+      tg = f32_target<SW>(a, tile);
+      load(tg, tile);
+    }
+    lds_barrier();
+    // lanes 0-31: the rows (gate), in group order; with SW lanes 32-63 the up rows (8 S <= 32)
+    if (tid < 64) {
+      const int r = tid & 31, sel = SW ? tid >> 5 : 0;
+      float v = 0.f;
+      if (r < S * RC) v = fold_chain(P + (sel * S * RC + r) * pst, nb);
+      const float up = SW ? __shfl_down(v, 32) : 0.f;
+      const int n = cur_tile * S * RC + r;
+      if (tid < 32 && r < S * RC && n < cur.N) {
+        if (SW) cur.y[n] = silu_exact(v) * up;
+        else cur.y[n] = (cur.res ? cur.res[n] : 0.f) + v;
+      }
+    }
+    if (at >= total) return;
+    lds_barrier();
+  }
+}
+
 // T == 1, q8, rows whose products fit the launch's 64 KB of LDS (x plus [sel][8 rows][4 chains][stride]
 // floats: K up to 1792 for one output, up to 768 for SwiGLU; longer rows take the four-lane kernels
 // below): the products x_i * w_i (each rounded, as dot_q8 forms
@@ -3050,6 +3167,7 @@ static int f32q4_tile_rows(int H, int nb, int nsel, int rows) {
 }
 
 bool f32act_q4_ok(int T, int K, int nb, int H, int nsel, int rows, bool norm) {
+  if (T == 1 && K == nb * kBlock && f32q4_wide_ok(nb, H)) return true;
   return T == 1 && H >= 1 && !(H & (H - 1)) && K == nb * kBlock &&
          f32q4_lds_bytes(K, nb, f32q4_tile_rows(H, nb, nsel, rows), nsel, norm) <= kMaxLds - 1024;
 }
@@ -3060,8 +3178,26 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
   int rows = 0;
   for (int i = 0; i < n; ++i) rows += a.tg[i].N;
   if (a.T == 1 && dtype == WQ4 && f32act_q4_ok(a.T, a.K, a.nb, a.H, nsel, rows, a.nw != nullptr)) {
-    // one workgroup per tile of rt rows; the tile starts counted in tiles here
     F32Args b = a;
+    if (f32q4_wide_ok(a.nb, a.H)) {
+      const int S = b.rt = f32q4_wide_sets(a.nb), pst = (((a.nb + 3) >> 2) | 1) << 2;
+      int tiles = 0;
+      for (int i = 0; i < n; ++i) {
+        b.tile_start[i] = tiles;
+        tiles += (a.tg[i].N + S * kF32QRows - 1) / (S * kF32QRows);
+      }
+      b.tile_start[n] = tiles;
+      if (tiles < 1) return hipErrorInvalidValue;
+      const int threads = a.nb <= 256 ? 256 : (a.nb + 63) & ~63;
+      const size_t lds = ((size_t)nsel * S * kF32QRows * pst + (a.nw ? 4 * (size_t)norm_rowlen(a.K) : 0)) * sizeof(float);
+      if (swiglu) b.tile_start[1] = tiles;
+      // about two workgroups per CU, each with the same number of tiles (the last ones perhaps one fewer)
+      const int per = (tiles + 511) / 512, grid = (tiles + per - 1) / per;
+      if (swiglu) gemv_f32act_q4_wide_kernel<true><<<grid, threads, lds, s>>>(b);
+      else gemv_f32act_q4_wide_kernel<false><<<grid, threads, lds, s>>>(b);
+      return hipGetLastError();
+    }
+    // one workgroup per tile of rt rows; the tile starts counted in tiles here
     const int rt = f32q4_tile_rows(a.H, a.nb, nsel, rows);
     b.rt = rt;
     int tiles = 0;
@@ -3128,13 +3264,14 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
     // The largest tile that makes at least two workgroups per CU (one for 32 rows x 16 tokens), else 16 rows x 8 tokens: at
     // 4096 x 4096 q4 and 256 / 128 / 64 / 32 / 16 tokens 64 x 32 tiles take 189 / 114 / 109 / 105 / 95 us, 64 x 16 220 / 115 /
     // 71 / 68 / 67, 32 x 16 240 / 124 / 65 / 41 / 40, 16 x 8 343 / 179 / 95 / 50 / 29. SwiGLU holds both selections, so at most
-    // 32 x 16 (3648 x 1088, 175 tokens, with its down projection: 148 us, 185 with 64 x 16).
+    // 32 x 16 (3648 x 1088, 175 tokens, with its down projection: 148 us, 185 with 64 x 16), and 16 x 8 up to 384 of those (1536 x
+    // 576 q8, 93 tokens, with its down projection: 35 against 42 us).
     auto wgs = [&](int ry, int tx) {
       int64_t g = 0;
       for (int i = 0; i < n; ++i) g += (a.tg[i].N + 16 * ry - 1) / (16 * ry);
       return g * ((a.T + kF32TWaves * tx - 1) / (kF32TWaves * tx));
     };
-    const int64_t big = 512, mid = 256;
+    const int64_t big = 512, mid = swiglu ? 384 : 256;
     auto go = [&](auto ry, auto tx, auto pp) {
       constexpr int RY = decltype(ry)::value, TX = decltype(tx)::value, P = decltype(pp)::value;
       F32Args b = a;

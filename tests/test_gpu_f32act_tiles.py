@@ -1,6 +1,6 @@
 """The f32-activation kernels at the sizes where their dispatch or tiles turn, bit for bit against the oracle: the LDS-tile
 GEMM's four tiles with ragged rows, tokens and row lengths (K past and short of whole 16s, 32s and 128s, K below 4), several
-targets."""
+targets, and the long-row one-token q4 GEMV with one and several row sets per workgroup, RMSNORM inside and outside."""
 import numpy as np
 import pytest
 
@@ -51,4 +51,36 @@ def test_f32act_gemm_rows_shorter_than_a_chain(ctx):
         x = r.normal(0, 1, (5, k)).astype(np.float32)
         d = up(ctx, w)
         assert bits_equal(ctx.matmul(x, [d], None, act=E.ACT_F32)[0], O.cpu_matmul(x, [w], None, act_quant=False)[0]), f"K={k}"
+        d.free()
+
+
+# (rows, K): 3, 2 and 1 row sets of a 256-thread workgroup, more than 256 groups, an odd number of groups
+WIDE = [(200, 2080), (90, 2720), (77, 4096), (100, 8192), (72, 8224), (41, 14336)]
+
+
+@pytest.mark.parametrize("shape", WIDE, ids=["x".join(map(str, s)) for s in WIDE])
+def test_f32act_long_row_gemv(ctx, shape):
+    n, k = shape
+    r = np.random.default_rng(n)
+    ws = [weight(r, n, k, O.Q4), weight(r, 24, k, O.Q4)]
+    wu = weight(r, n, k, O.Q4)
+    dws, du = [up(ctx, w) for w in ws], up(ctx, wu)
+    x = r.normal(0, 1, (1, k)).astype(np.float32)
+    res = r.normal(0, 1, (1, n)).astype(np.float32)
+    print(f"[gpu] f32act long rows {n}x{k}", flush=True)
+    got = ctx.matmul(x, dws, [res, None], act=E.ACT_F32)
+    for g, w in zip(got, O.cpu_matmul(x, ws, [res, None], act_quant=False)):
+        assert bits_equal(g, w)
+    assert bits_equal(ctx.swiglu(x, dws[0], du, act=E.ACT_F32), O.cpu_swiglu(x, ws[0], wu, act_quant=False))
+    if k <= 8192:  # RMSNORM in the call
+        nw = r.normal(1, 0.1, k).astype(np.float32)
+        xn = O.rmsnorm(x, nw, 1e-5)
+        bx, bn, by = ctx.buffer(x.nbytes).upload(x), ctx.buffer(nw.nbytes).upload(nw), ctx.buffer(n * 4)
+        ctx.rmsnorm_matmul_dev(bx.ptr, bn.ptr, 1e-5, 1, k, [dws[0]], [by.ptr], None, act=E.ACT_F32)
+        assert bits_equal(by.download((1, n), np.float32), O.cpu_matmul(xn, [ws[0]], None, act_quant=False)[0])
+        ctx.rmsnorm_swiglu_dev(bx.ptr, bn.ptr, 1e-5, 1, k, dws[0], du, by.ptr, act=E.ACT_F32)
+        assert bits_equal(by.download((1, n), np.float32), O.cpu_swiglu(xn, ws[0], wu, act_quant=False))
+        for b in (bx, bn, by):
+            b.free()
+    for d in dws + [du]:
         d.free()
