@@ -1829,6 +1829,189 @@ __global__ __launch_bounds__(256) void gemm_wave16_kernel(const GemmArgs a) {
   wave16_store<WDT, SW, TOK>(a, tg, r0, t0, lane, iacc, facc);
 }
 
+// A few tokens over long rows (K > 1536): one wave per 16 x 16 tile left a SIMD with one wave or none, walking all of K
+// through one serial rescale (down 4096 x 14336 q4, 16 tokens: 256 waves, 99 us). Here a workgroup of eight waves shares a
+// 16-row x 16-token tile (gate and up with SW) and splits K: a round is 8 G blocks, each wave takes G of them, one MFMA
+// each, and leaves the blocks' rescaled products in LDS (block, lane: 16 bytes, no bank conflicts); behind the next barrier
+// further waves, one lane per output, add the round's products in block order while the next round is made, so the f32 sums
+// are the other kernels', bit for bit. The operands come by DMA, 1 KB per instruction, in a ring of D slots; one barrier per
+// round covers the ring, the products and the fold (SwiGLU has room for one product buffer, and two barriers). Per-token q8
+// sums are integers: every wave accumulates its share in the MFMA and the eight are added once. Bound by what the CUs pull
+// from L2 (900 bytes per block and tile, 512 of them activations that every row tile reads again: 8.4 TB/s at 128 tokens).
+// Operands loaded straight into registers (four instructions per block and wave) took 75 against 57 us at 64 tokens.
+constexpr int kSplitWaves = 8;  // producer waves; one more per 64 outputs folds
+template <int WDT, bool SW, bool TOK, int G, int D>
+struct SplitLds {  // a ring slot: activations [RB blocks][2 halves][16 tokens][16 bytes], weights [sel][RB][16 rows][32 or 16
+                   // bytes], q4 scales [sel][RB][16], block scales [RB][16 tokens]
+  static constexpr int RB = kSplitWaves * G, NSEL = SW ? 2 : 1, WK = WDT == WQ8 ? RB / 2 : RB / 4, CK = RB / 16;  // WK, CK: KB
+  static constexpr int W = RB / 2, C = W + NSEL * WK, XD = C + (WDT == WQ4 ? NSEL * CK : 0), KB = XD + (TOK ? 0 : CK);
+  static constexpr int PER_WAVE = (KB + kSplitWaves - 1) / kSplitWaves;  // 1 KB DMA instructions of a round per producer
+  static constexpr bool INT = TOK && WDT == WQ8;
+  static constexpr int NP = SW ? 1 : 2;  // product buffers
+  static constexpr int PROD = (INT ? kSplitWaves : NP * RB) * NSEL * 1024;
+  static constexpr int BYTES = D * KB * 1024 + PROD, WAVES = kSplitWaves + (INT ? 0 : 4 * NSEL);
+};
+template <int WDT, bool SW, bool TOK, int G, int D>
+__global__ __launch_bounds__((64 * SplitLds<WDT, SW, TOK, G, D>::WAVES)) void gemm_split16_kernel(const GemmArgs a) {
+  typedef SplitLds<WDT, SW, TOK, G, D> L;
+  constexpr int NSEL = L::NSEL, RB = L::RB, PW = L::PER_WAVE, NP = L::NP;
+  constexpr bool INT = L::INT;
+  extern __shared__ __align__(16) unsigned char split_lds[];
+  v4i* const P = reinterpret_cast<v4i*>(split_lds + D * L::KB * 1024);  // [NP][NSEL][RB][64]
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, c4 = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nb = a.nb, H = a.H, lgH = __builtin_ctz(H), ngroups = (a.T + kWave16 - 1) / kWave16;
+  // workgroup -> (target, 16-row tile, 16-token group): eight row tiles side by side, then the next token group, so that the
+  // workgroups that share weight rows run close together on one XCD (workgroup index mod 8)
+  const int oct = (int)blockIdx.x / (8 * ngroups), in = (int)blockIdx.x - oct * 8 * ngroups;
+  const int g = in >> 3;
+  int rt = 8 * oct + (in & 7);
+  int ti = 0;
+  const int n = SW ? 1 : a.n_targets;
+  for (; ti < n; ++ti) {
+    const int cnt = (a.tg[ti].N + kWave16 - 1) / kWave16;
+    if (rt < cnt) break;
+    rt -= cnt;
+  }
+  if (ti >= n) return;  // past the last tile (the whole workgroup)
+  const GemmTarget tg = SW ? a.tg[0] : gemm_target_at(ti);
+  const int r0 = rt * kWave16, t0 = g * kWave16;
+  const unsigned lds0 = (unsigned)(size_t)(LdsBytes)split_lds;
+  // item (row r0 + r, block b) of the weight layout; rows past N: padding (rows_pad is a multiple of 64)
+  auto item = [&](int r, int b) { return ((((r0 + r) >> lgH) * nb + b) << lgH) + ((r0 + r) & (H - 1)); };
+  // the round's operands into its slot: instruction id = w + 8 i copies kilobyte id of the slot (blocks past the row's last
+  // repeat it: their products are dropped)
+  auto request = [&](int r) __attribute__((always_inline)) {
+    const unsigned slot = lds0 + (unsigned)(r % D) * (L::KB * 1024);
+    const int b0 = r * RB;
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const int id = w + kSplitWaves * i < L::KB ? w + kSplitWaves * i : w;  // spare: the wave's first one again
+      const unsigned dst = slot + id * 1024;
+      if (id < L::W) {  // activations: chunk (block, half, token)
+        const int j = 64 * id + lane, b = min(b0 + (j >> 5), nb - 1);
+        dma16s(a.xq, (uint32_t)((((t0 >> 5) * nb + b) << 10) + (((j >> 4) & 1) << 9) + ((t0 & 31) + (j & 15)) * 16), dst);
+      } else if (id < L::C) {
+        const int k = id - L::W, s = k / L::WK, j = 64 * (k % L::WK) + lane;
+        const uint8_t* const data = SW && s ? a.tg[1].data : tg.data;
+        if (WDT == WQ8)  // chunk (block, row, 16-byte half)
+          dma16s(data, (uint32_t)item((j >> 1) & 15, min(b0 + (j >> 5), nb - 1)) * 32u + (j & 1) * 16u, dst);
+        else
+          dma16s(data, (uint32_t)item(j & 15, min(b0 + (j >> 4), nb - 1)) * 16u, dst);
+      } else if (WDT == WQ4 && id < L::XD) {  // q4 scales: chunk (block, four rows)
+        const int k = id - L::C, s = k / L::CK, j = 64 * (k % L::CK) + lane;
+        dma16s(SW && s ? a.tg[1].scales : tg.scales, (uint32_t)item((j & 3) * 4, min(b0 + (j >> 2), nb - 1)) * 4u, dst);
+      } else if (!TOK) {  // block scales: chunk (block, four tokens)
+        const int j = 64 * (id - L::XD) + lane;
+        dma16s(a.xd, (uint32_t)(min(b0 + (j >> 2), nb - 1) * a.Tpad + t0 + (j & 3) * 4) * 4u, dst);
+      }
+    }
+  };
+  const int nr = (nb + RB - 1) / RB;
+  const v4i zero = {0, 0, 0, 0};
+  v4i isum[NSEL];
+#pragma unroll
+  for (int s = 0; s < NSEL; ++s) isum[s] = zero;
+  float acc = 0.f;
+  // the fold: four waves per selection after the producers (per-token q8: the first ones, once)
+  const int fw = INT ? w : w - kSplitWaves, sel = SW ? (fw >> 2) & 1 : 0;
+  const bool folds = fw >= 0 && fw < 4 * NSEL, makes = w < kSplitWaves;
+  auto produce = [&](int r) __attribute__((always_inline)) {
+    const unsigned char* const slot = split_lds + (r % D) * (L::KB * 1024);
+    v4i* const pr = P + (r & (NP - 1)) * (NSEL * RB * 64);
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      const int j = w * G + k;
+      const long A = *reinterpret_cast<const long*>(slot + j * 512 + (c4 >> 1) * 256 + l16 * 16 + (c4 & 1) * 8);
+      float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (!TOK) xv = *reinterpret_cast<const float4*>(slot + L::XD * 1024 + j * 64 + c4 * 16);
+      const bool in_row = r * RB + j < nb;
+#pragma unroll
+      for (int s = 0; s < NSEL; ++s) {
+        const unsigned char* const wp = slot + (L::W + s * L::WK) * 1024;
+        const long B = WDT == WQ8 ? *reinterpret_cast<const long*>(wp + (j * 16 + l16) * 32 + c4 * 8)
+                                  : q4_operand8(*reinterpret_cast<const uint2*>(wp + (j * 16 + l16) * 16 + (c4 & 1) * 8), c4 >> 1);
+        if (INT) {
+          if (in_row) isum[s] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B, isum[s], 0, 0, 0);
+        } else {
+          const float c = WDT == WQ4 ? *reinterpret_cast<const float*>(slot + (L::C + s * L::CK) * 1024 + (j * 16 + l16) * 4) : 1.f;
+          const v4i S = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B, zero, 0, 0, 0);
+          const float x4[4] = {xv.x, xv.y, xv.z, xv.w};
+          v4i p;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            // as gemm_wave16_kernel: q8 float(S) * xd; q4 (S = 16 * S_b) float(S) * (ws * xd), 16 times edgelm's product
+            const float m = TOK ? c : WDT == WQ8 ? x4[i] : c * x4[i];
+            p[i] = in_row ? __float_as_int((float)S[i] * m) : 0;  // +0.0 changes no sum
+          }
+          pr[(s * RB + j) * 64 + lane] = p;
+        }
+      }
+    }
+  };
+  auto fold = [&](int r) __attribute__((always_inline)) {
+    const float* const col = reinterpret_cast<const float*>(P + ((r & (NP - 1)) * NSEL + sel) * (RB * 64)) + (fw & 3) * 64 + lane;
+    float v[RB];
+#pragma unroll
+    for (int j = 0; j < RB; ++j) v[j] = col[256 * j];
+#pragma unroll
+    for (int j = 0; j < RB; ++j) acc = acc + v[j];
+  };
+  if (makes) {
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) request(d);
+  }
+  for (int r = 0; r < nr; ++r) {
+    if (makes) wait_vm<(D - 2) * PW>();  // this wave's part of round r has landed
+    // every wave's part has; round r - 1's products are in LDS, its slot is free, and earlier products have been added
+    lds_barrier();
+    if (makes) {
+      request(r + D - 1);  // past the last round too (the last block again): the wait's count stays the same
+      produce(r);
+    } else if (NP == 2 && r > 0) {
+      fold(r - 1);
+    }
+    if (NP == 1 && !INT) {
+      lds_barrier();
+      if (!makes) fold(r);
+    }
+  }
+  wait_vm<0>();  // no copy outlives the workgroup's LDS
+  // output o = (fw & 3) * 64 + lane of a selection: row o / 4 % 16, token 4 (o / 64) + o % 4
+  if (INT) {
+#pragma unroll
+    for (int s = 0; s < NSEL; ++s) P[(s * kSplitWaves + w) * 64 + lane] = isum[s];
+  }
+  lds_barrier();
+  if (INT) {
+    int S = 0;
+    if (folds) {
+      const int* const col = reinterpret_cast<const int*>(P + sel * (kSplitWaves * 64)) + (fw & 3) * 64 + lane;
+#pragma unroll
+      for (int j = 0; j < kSplitWaves; ++j) S += col[256 * j];
+    }
+    acc = (float)S;
+  } else if (NP == 2 && folds) {
+    fold(nr - 1);
+  }
+  const int o = (fw & 3) * 64 + lane, row = r0 + ((o >> 2) & 15), t = t0 + 4 * (o >> 6) + (o & 3);
+  float v;
+  {
+    const float xt = TOK ? a.xd[min(t, a.Tpad - 1)] : 1.f;
+    const float ws = WDT == WQ8 ? (SW && sel ? a.tg[1].scales : tg.scales)[min(row, tg.N - 1)] : 1.f;
+    if (WDT == WQ8) v = TOK ? (acc * xt) * ws : acc * ws;
+    else v = TOK ? (acc * 0.0625f) * xt : acc * 0.0625f;
+  }
+  if (SW) {
+    float* const ex = reinterpret_cast<float*>(split_lds);  // the ring is drained and read
+    if (folds && sel) ex[o] = v;
+    lds_barrier();
+    if (folds && !sel && row < tg.N && t < a.T) tg.y[(int64_t)t * tg.N + row] = silu_exact(v) * ex[o];
+  } else if (folds && row < tg.N && t < a.T) {
+    tg.y[(int64_t)t * tg.N + row] = tg.res ? v + tg.res[(int64_t)t * tg.N + row] : v;
+  }
+}
+
 // Small GEMMs (K <= 1536: the prefill of a small model): gemm_wave16_kernel's waves and arithmetic
 // (the same bits), with a workgroup's operands (one 16-row tile, 64 tokens: four waves of 16
 // tokens) moved into LDS by DMA in one go, 1 KB per instruction, every request out before the
@@ -3033,6 +3216,38 @@ static void gemm_wave16_launch(const GemmArgs& a, hipStream_t s) {
     gemm_wave16_kernel<WDT, SW, TOK, false><<<grid, 256, 0, s>>>(a);
 }
 
+template <bool SW>
+static int64_t gemm_split16_wgs(const GemmArgs& a) {
+  int64_t rows = 0;
+  for (int i = 0; i < (SW ? 1 : a.n_targets); ++i) rows += (a.tg[i].N + kWave16 - 1) / kWave16;
+  return (rows + 7) / 8 * 8 * ((a.T + kWave16 - 1) / kWave16);
+}
+template <int WDT, bool SW, bool TOK>
+static hipError_t gemm_split16_launch(const GemmArgs& a, hipStream_t s) {
+  if (gemm_split16_wgs<SW>(a) > INT32_MAX) return hipErrorInvalidValue;
+  const int wgs = (int)gemm_split16_wgs<SW>(a);
+  auto go = [&](auto gg, auto d) {
+    constexpr int G = decltype(gg)::value, D = decltype(d)::value;
+    typedef SplitLds<WDT, SW, TOK, G, D> L;
+    if (L::BYTES > 64 * 1024) {
+      static const hipError_t raised = hipFuncSetAttribute((const void*)gemm_split16_kernel<WDT, SW, TOK, G, D>,
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, L::BYTES);
+      if (raised != hipSuccess) return raised;
+    }
+    gemm_split16_kernel<WDT, SW, TOK, G, D><<<wgs, 64 * L::WAVES, L::BYTES, s>>>(a);
+    return hipGetLastError();
+  };
+  // one workgroup per CU: longer rounds (q4 4096 x 14336, 16 tokens 22.1 against 23.9 us), or for the per-token sums one more
+  // slot (18.6 against 23.7 us); more: two slots of 16 blocks, so that two workgroups fit a CU (64 tokens 57 us; 70 with the
+  // longer rounds, 59 with three slots)
+  using std::integral_constant;
+  if (wgs <= 256) {
+    if constexpr (TOK && WDT == WQ8) return go(integral_constant<int, 2>{}, integral_constant<int, 3>{});
+    else if constexpr (!SW) return go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+  }
+  return go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+}
+
 // gemm_lds16_kernel when its LDS fits (K <= 1536 or so); false otherwise
 template <int WDT, bool SW, bool TOK, bool QF = false>
 static bool gemm_lds16_launch(const GemmArgs& a, hipStream_t s) {
@@ -3123,6 +3338,16 @@ static hipError_t gemm_go(const GemmArgs& a, int tiles, hipStream_t s) {
     wave32 = std::strcmp(ev, "wave32") == 0;
     lds16 = ev[0] == 'l';
   }
+  // A few tokens over long rows: K split over a workgroup's waves (gemm_split16_kernel) up to 2048 workgroups, 1200 with
+  // SwiGLU (each the work of two). Per-block q4, against the kernels below: 4096 x 14336 at 16 / 64 / 128 / 256 tokens (256 /
+  // 1024 / 2048 / 4096 workgroups) 22 / 57 / 103 / 214 us against 104 / 95 / 123 / 136; 4096 x 4096 10 / 21 / 35 / 69 against
+  // 32 / 32 / 38 / 44; 14336 x 4096 at 16 / 32 / 64 tokens 21 / 34 / 62 against 33 / 39 / 64. ELMH_GEMM_KERNEL=split forces
+  // it. Not for the fused multiply-adds of ELMH_FAST.
+  const int64_t split_wgs = gemm_split16_wgs<SW>(a);
+  const char* const forced = getenv("ELMH_GEMM_KERNEL");
+  const bool split = forced ? std::strcmp(forced, "split") == 0
+                            : a.nb > kLds16MaxBlocks && split_wgs <= (SW ? 1200 : 2048) && !getenv("ELMH_GEMM_TOKEN_TILE");
+  if (split && !a.fast && a.H >= 4 && !(a.H & (a.H - 1))) return gemm_split16_launch<WDT, SW, TOK>(a, s);
   if (wave) {
     if (wave32)
       gemm_wave_launch<WDT, SW, TOK>(a, s);
