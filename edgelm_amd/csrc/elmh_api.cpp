@@ -373,7 +373,7 @@ int quant_frag(elmh_ctx* c, const Scratch& sc, const float* x, int T, int64_t K,
   return ELMH_OK;
 }
 
-// RMSNORM and the block-scale fragment quantization in one launch (K <= 2048)
+// RMSNORM and the block-scale fragment quantization in one launch (K <= 8192)
 int quant_frag_norm(elmh_ctx* c, const float* x, const float* nw, float eps, int T, int64_t K, int* Tpad_out,
                     ActBufs* a) {
   const int Tpad = (int)round_up(T, kGemmTileT);
@@ -513,7 +513,7 @@ int run_swiglu(elmh_ctx* c, const float* x, int T, int64_t K, const elmh_weight*
   }
   const bool qin = use_small_gemv(T, K, g.data_bytes + g.scale_bytes + u.data_bytes + u.scale_bytes);
   const int nt = gemv_tokens(g, 2, qin);
-  if (nw && !(act == ELMH_ACT_INT8 && (T <= nt ? qin : K <= 2048)))
+  if (nw && !(act == ELMH_ACT_INT8 && (T <= nt ? qin : K <= 8192)))
     return fail(c, ELMH_ERR_UNSUPPORTED, "swiglu: fused rmsnorm off the small GEMV and block-scale GEMM paths");
   if (act == ELMH_ACT_INT8 && T <= nt) {
     GemvArgs a{};
@@ -626,7 +626,7 @@ bool f32_norm_fusable(int T, int64_t K, int n, const elmh_weight* const* w, int 
 }
 
 bool norm_gemm(int T, int64_t K, int n, const elmh_weight* const* w, int nsel, int act) {
-  return K <= 2048 && block_gemm(T, K, n, w, nsel, act);
+  return K <= 8192 && block_gemm(T, K, n, w, nsel, act);
 }
 
 // RMSNORM into the scratch buffer (the path when it cannot be fused)

@@ -147,23 +147,27 @@ __global__ __launch_bounds__(256) void act_quant_frag_kernel(const float* __rest
 }
 
 // RMSNORM and the GEMM's per-block activation quantization in one pass (the input of a layer's
-// QKV and gate/up GEMMs): kNqTok rows per workgroup, each normalized in rmsnorm_kernel's order
+// QKV and gate/up GEMMs): NQ rows per workgroup, each normalized in rmsnorm_kernel's order
 // (squares grouped by dot_f32_scalar's accumulators in LDS, four in-order sums, (s0 + s1) +
 // (s2 + s3), then (x * inv) * w), then quantized into fragments exactly as act_quant_frag_kernel
 // does. A thread owns up to kNqItems half-blocks (row, block, half) and loads their x and norm
 // weights at the start, so the normalized values never leave its registers; the two halves of a
-// block sit in neighbouring lanes. Tokens at or past T give zero fragments and scales. K <= 2048.
-constexpr int kNqTok = 4;
-constexpr int kNqItems = 2;  // kNqTok * (2048 / 32) * 2 half-blocks over 256 threads
+// block sit in neighbouring lanes. Tokens at or past T give zero fragments and scales.
+// NQ = 4 up to K = 2048 and 1 up to K = 8192: the half-blocks of a workgroup's rows fill its
+// threads' items either way. The in-order sums of K / 4 squares bound it. At K = 4096 one launch
+// takes 8.3 us for 16 tokens and 11.9 us for 333; RMSNORM and the quantizer in launches of their
+// own took 9.0 + 4.9 and 9.1 + 5.6 us.
+constexpr int kNqItems = 2;  // 4 * (2048 / 32) * 2 or (8192 / 32) * 2 half-blocks over 256 threads
 
+template <int NQ>
 __global__ __launch_bounds__(256) void rmsnorm_quant_frag_kernel(const float* __restrict__ x, const float* __restrict__ nw,
                                                                  float eps, int T, int Tpad, int K,
                                                                  int8_t* __restrict__ xq, float* __restrict__ xd) {
   extern __shared__ __align__(16) float nq_lds[];
-  __shared__ float inv_l[kNqTok];
+  __shared__ float inv_l[NQ];
   const int K4 = K >> 2, rowlen = norm_rowlen(K), nb = K / kBlock;
-  float* sq = nq_lds;  // [kNqTok][4][rowlen]
-  const int t0 = blockIdx.x * kNqTok, tid = threadIdx.x, items = kNqTok * nb * 2;
+  float* sq = nq_lds;  // [NQ][4][rowlen]
+  const int t0 = blockIdx.x * NQ, tid = threadIdx.x, items = NQ * nb * 2;
   float4 xv[kNqItems][4], wv[kNqItems][4];
 #pragma unroll
   for (int i = 0; i < kNqItems; ++i) {
@@ -187,23 +191,25 @@ __global__ __launch_bounds__(256) void rmsnorm_quant_frag_kernel(const float* __
       }
     }
   }
-  // +0.0 up to the next multiple of 16 terms
-  for (int i = tid; i < kNqTok * 4 * 16; i += 256)
-    if (K4 + (i & 15) < ((K4 + 15) & ~15)) sq[(i >> 4) * rowlen + K4 + (i & 15)] = 0.f;
-  __syncthreads();
-  if (tid < 4 * kNqTok) {
-    const float sacc = ordered_sum(sq + tid * rowlen, K4, 0.f);
-    const float s01 = sacc + dpp_f<kDppQuadXor1>(sacc);
-    const float ss = s01 + dpp_f<kDppQuadXor2>(s01);
-    if ((tid & 3) == 0) inv_l[tid >> 2] = 1.0f / sqrtf(ss / (float)K + eps);
+  if (t0 < T) {  // a workgroup of token slots past T needs no sums
+    // +0.0 up to the next multiple of 16 terms
+    for (int i = tid; i < NQ * 4 * 16; i += 256)
+      if (K4 + (i & 15) < ((K4 + 15) & ~15)) sq[(i >> 4) * rowlen + K4 + (i & 15)] = 0.f;
+    __syncthreads();
+    if (tid < 4 * NQ) {
+      const float sacc = ordered_sum(sq + tid * rowlen, K4, 0.f);
+      const float s01 = sacc + dpp_f<kDppQuadXor1>(sacc);
+      const float ss = s01 + dpp_f<kDppQuadXor2>(s01);
+      if ((tid & 3) == 0) inv_l[tid >> 2] = 1.0f / sqrtf(ss / (float)K + eps);
+    }
+    __syncthreads();
   }
-  __syncthreads();
 #pragma unroll
   for (int i = 0; i < kNqItems; ++i) {
     const int it = tid + 256 * i;
     if (it < items) {  // items is even: both lanes of a block pair take this branch
       const int r = it / (2 * nb), rem = it - r * 2 * nb, b = rem >> 1, h = rem & 1, t = t0 + r;
-      const float inv = inv_l[r];
+      const float inv = t0 < T ? inv_l[r] : 0.f;
       float4 v[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -3009,10 +3015,12 @@ hipError_t launch_act_quant_frag(const float* x, int T, int Tpad, int K, int8_t*
 
 hipError_t launch_rmsnorm_quant_frag(const float* x, const float* nw, float eps, int T, int Tpad, int K, int8_t* xq,
                                      float* xd, hipStream_t s) {
-  if (K % kBlock || K > 2048 || Tpad % kNqTok) return hipErrorInvalidValue;
-  const size_t rowlen = (size_t)norm_rowlen(K);
-  const size_t lds = (size_t)kNqTok * 4 * rowlen * sizeof(float);
-  rmsnorm_quant_frag_kernel<<<Tpad / kNqTok, 256, lds, s>>>(x, nw, eps, T, Tpad, K, xq, xd);
+  if (K % kBlock || K > 8192 || Tpad % 4) return hipErrorInvalidValue;
+  const size_t lds = 4 * (size_t)norm_rowlen(K) * sizeof(float);
+  if (K <= 2048)
+    rmsnorm_quant_frag_kernel<4><<<Tpad / 4, 256, 4 * lds, s>>>(x, nw, eps, T, Tpad, K, xq, xd);
+  else
+    rmsnorm_quant_frag_kernel<1><<<Tpad, 256, lds, s>>>(x, nw, eps, T, Tpad, K, xq, xd);
   return hipGetLastError();
 }
 

@@ -166,7 +166,7 @@ int elmh_rmsnorm_dev(elmh_ctx* ctx, const float* x, const float* w, float* y, in
  * (passes.cpp:72-81,100-104; cpu::rmsnorm kernels_cpu.cpp:326-335). With int8 activations on
  * rows short enough for the workgroup-quantizing GEMV (T <= 4, K <= 2048) each workgroup
  * normalizes the rows itself and the normalized activation never goes to memory; on the
- * block-scale GEMM path (K <= 2048) one launch normalizes and quantizes the rows into the GEMM's
+ * block-scale GEMM path one launch normalizes and quantizes the rows into the GEMM's
  * operand; otherwise the normalized rows go to a scratch buffer (reserved by elmh_reserve)
  * first. K <= 8192. */
 int elmh_rmsnorm_matmul_dev(elmh_ctx* ctx, const float* x, const float* norm_w, float eps, int T, int64_t K,
