@@ -53,9 +53,8 @@ ELM_HOSTDEV static inline uint64_t elm_exp2_tab(uint32_t i) {
   return elm_d2u(y) - ((kElmExp2Fix >> i) & 1u) - ((uint64_t)i << 47);
 }
 
-// expf with the table entry for i from entry(i): elm_exp2_tab itself, or a copy of its 32 values
-template <class Entry>
-ELM_HOSTDEV static inline float elm_expf_by(float x, Entry entry) {
+// expf with the table entries from elm_exp2_tab, or (from_tab, a constant at each call) from a copy of its 32 values
+ELM_HOSTDEV static inline float elm_expf_by(float x, const uint64_t* tab, int from_tab) {
   const uint32_t ux = elm_f2u(x);
   const uint32_t abstop = (ux >> 20) & 0x7ff;
   if (abstop >= 0x42b) {                         // |x| >= 88 (top 12 bits of 88.0f), or inf/nan
@@ -74,7 +73,7 @@ ELM_HOSTDEV static inline float elm_expf_by(float x, Entry entry) {
   const uint64_t ki = elm_d2u(kd);
   kd -= shift;
   const double r = __builtin_fma(inv_ln2_n, xd, -kd);
-  const uint64_t t = entry((uint32_t)(ki & 31)) + (ki << 47);
+  const uint64_t t = (from_tab ? tab[ki & 31] : elm_exp2_tab((uint32_t)(ki & 31))) + (ki << 47);
   const double s = elm_u2d(t);
   const double z = __builtin_fma(c0, r, c1);
   const double r2 = r * r;
@@ -84,12 +83,8 @@ ELM_HOSTDEV static inline float elm_expf_by(float x, Entry entry) {
   return (float)y;
 }
 
-ELM_HOSTDEV static inline float elm_expf(float x) {
-  return elm_expf_by(x, [](uint32_t i) { return elm_exp2_tab(i); });
-}
+ELM_HOSTDEV static inline float elm_expf(float x) { return elm_expf_by(x, 0, 0); }
 
 // The same value with the 32 table entries read from memory (a workgroup's LDS, filled with elm_exp2_tab): an LDS read
 // instead of the 13 double-precision steps of the polynomial, for kernels that take many exponentials per thread.
-ELM_HOSTDEV static inline float elm_expf_tab(float x, const uint64_t* tab) {
-  return elm_expf_by(x, [tab](uint32_t i) { return tab[i]; });
-}
+ELM_HOSTDEV static inline float elm_expf_tab(float x, const uint64_t* tab) { return elm_expf_by(x, tab, 1); }
