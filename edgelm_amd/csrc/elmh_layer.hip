@@ -1333,11 +1333,14 @@ __global__ __launch_bounds__(256) void attention_rows_kernel(const float* __rest
 // every phase that is not one ordered chain is spread over 16 waves:
 //  - scores as in attention_rows_kernel: a lane per position, 64 positions per wave and 1024 per pass, 16 dims of a wave's
 //    key rows at a time through a 4 KB LDS piece of its own, the query broadcast by the multiply;
-//  - the in-order sum of the exponentials on wave 0 while the waves that will add the values request the first 64 positions;
-//  - output: a lane per dim, four batches of 16 positions in flight (one position's values are one coalesced request).
+//  - the in-order sum of the exponentials on wave 0 while the waves that will add the values request the first 64 positions
+//    and the other waves touch the rest, so that it comes from this XCD's L2 later;
+//  - output: a lane per dim, four batches of 16 positions in flight (one position's values are one coalesced request). A wave
+//    that adds issues one instruction in some 5 clocks, so the loop is their count: 3.9 per position with the rows' offsets in
+//    scalar registers against 9.1 with a clamped address each (700 positions 22 -> 17 us, 1900 54 -> 38 us).
 // The step's own key (rotated) replaces its row of the piece in LDS and its value is added last from a register, as the kv
 // group's first workgroup is still writing them to the cache.
-// 32 heads over 8 kv heads, head size 128, 700 cached positions: 22 us against 44 us with attention_kernel.
+// 32 heads over 8 kv heads, head size 128, 700 cached positions: 17 us against 44 us with attention_kernel.
 // LDS (dynamic): scores [n_cap rounded up to 16, and 256 more that reads ahead may touch], key pieces [16][64][16], query and
 // step's key [16 ceil(hd / 16)] each.
 constexpr int kStepWaves = 16;
@@ -1473,6 +1476,15 @@ __global__ __launch_bounds__(64 * kStepWaves) void attention_step_kernel(
 #pragma unroll
     for (int u = 0; u < 16; ++u) b[u] = vd[(int64_t)min(j0 + u, rlast) * hd];
   };
+  // the same for 16 positions that are all cached: one instruction each, the row's offset in a scalar register (the clamped
+  // addresses are five more per position, which is what bounds a wave that adds)
+  const uint32_t rowb = (uint32_t)hd * 4u, voff = (uint32_t)dc * 4u;
+  auto load_full = [&](int j0, float (&b)[16]) {
+    const __amdgpu_buffer_rsrc_t rv =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vh) + (int64_t)j0 * hd, (short)0, (int)(16u * rowb), 0x00020000);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) b[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, voff, u * rowb, 0));
+  };
   if (w == 0) {
     float sum = 0.f;
     for (int g0 = 0; g0 < n16; g0 += 256) sum = ordered_sum256(sc + g0, min(16, (n16 - g0) >> 4), sum);
@@ -1483,6 +1495,15 @@ __global__ __launch_bounds__(64 * kStepWaves) void attention_step_kernel(
     load(16, v[1]);
     load(32, v[2]);
     load(48, v[3]);
+  } else {
+    // the rest of the value rows into this XCD's L2, one load per 128-byte line
+    const int first = 1 + ((hd + 63) >> 6), step = 64 * (kStepWaves - first) * 32, end = nc * hd;
+    for (int f = 64 * hd + 32 * (64 * (w - first) + lane); f < end; f += 4 * step) {
+      float a[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a[u] = vh[f + u * step < end ? f + u * step : f];
+      asm volatile("" ::"v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
+    }
   }
   lds_barrier();  // the values stay in flight
   if (!adds) return;
@@ -1501,7 +1522,17 @@ __global__ __launch_bounds__(64 * kStepWaves) void attention_step_kernel(
   };
 #undef ELM_OUT_STEP
   int j0 = 0;
-  for (; j0 + 64 <= nc; j0 += 64) {
+  for (; j0 + 128 <= nc; j0 += 64) {
+    batch(j0, v[0], true);
+    load_full(j0 + 64, v[0]);
+    batch(j0 + 16, v[1], true);
+    load_full(j0 + 80, v[1]);
+    batch(j0 + 32, v[2], true);
+    load_full(j0 + 96, v[2]);
+    batch(j0 + 48, v[3], true);
+    load_full(j0 + 112, v[3]);
+  }
+  if (j0 + 64 <= nc) {
     batch(j0, v[0], true);
     load(j0 + 64, v[0]);
     batch(j0 + 16, v[1], true);
@@ -1510,6 +1541,7 @@ __global__ __launch_bounds__(64 * kStepWaves) void attention_step_kernel(
     load(j0 + 96, v[2]);
     batch(j0 + 48, v[3], true);
     load(j0 + 112, v[3]);
+    j0 += 64;
   }
   if (j0 < nc) batch(j0, v[0], false);
   if (j0 + 16 < nc) batch(j0 + 16, v[1], false);

@@ -69,3 +69,29 @@ def test_chunk_attention_writes_the_gemm_operand(ctx, T):
     for b in bufs:
         b.free()
     dw.free()
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(4, 2, 128), (3, 1, 100), (2, 1, 256), (4, 4, 16)])
+def test_step_attention_bit_exact(ctx, nh, nkv, hd):
+    """One token, its position in device memory, around the 16-, 64- and 1024-position steps and the 64 value rows in flight;
+    the cache past the step's position is NaN."""
+    mc = 1200
+    r = np.random.default_rng(hd + mc)
+    tab = O.rope_table(hd, mc, 10000.0)
+    up = lambda a: ctx.buffer(a.nbytes).upload(a)  # noqa: E731
+    for pos in (0, 1, 15, 16, 63, 64, 65, 127, 128, 129, 191, 192, 700, 1023, 1024, 1100):
+        kc, vc = (r.normal(0, 1, (nkv, mc, hd)).astype(np.float32) for _ in range(2))
+        kc[:, pos:], vc[:, pos:] = np.nan, np.nan
+        q = r.normal(0, 1, (1, nh * hd)).astype(np.float32)
+        k, v = (r.normal(0, 1, (1, nkv * hd)).astype(np.float32) for _ in range(2))
+        bufs = [up(a) for a in (q, k, v, kc, vc, *tab, np.array([pos], np.int32))] + [ctx.buffer(q.nbytes)]
+        bq, bk, bv, bkc, bvc, bc, bs, bp, bo = bufs
+        print(f"[gpu] step attention {nh, nkv, hd, mc} position {pos}", flush=True)
+        ctx.attention_step_dev(bq.ptr, bk.ptr, bv.ptr, bo.ptr, bp.ptr, nh, nkv, hd, bkc.ptr, bvc.ptr, mc, bc.ptr, bs.ptr)
+        want = O.attention(q, k, v, pos, nh, nkv, kc, vc, tab)
+        assert bits_equal(bo.download(q.shape, np.float32), want)
+        n = pos + 1
+        assert bits_equal(bkc.download(kc.shape, np.float32)[:, :n], kc[:, :n])
+        assert bits_equal(bvc.download(vc.shape, np.float32)[:, :n], vc[:, :n])
+        for b in bufs:
+            b.free()
