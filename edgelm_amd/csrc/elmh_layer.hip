@@ -1120,9 +1120,11 @@ __global__ __launch_bounds__(256) void attention_prefill64_kernel(
 //  - softmax: 256 / R lanes per row; the exponentials' table in LDS; the in-order sum in every lane of the row at once.
 //  - output: a lane holds one dim of R / (2 RS) rows (a wave 32 dims, its two halves different rows; RS = 2 splits the
 //    rows over two pairs of waves where two waves cover the dims); values come straight from the cache, 16 positions per
-//    batch, the next batch in flight; p_j = e_j * inv of 16 positions lies in 16 lanes and is broadcast by the multiply.
+//    batch, the next batch in flight; p_j = e_j * inv of 16 positions lies in 16 lanes and is broadcast by the multiply. Where
+//    all of a batch's positions are below nmax a load is one instruction, the row's offset in a scalar register (with a clamped
+//    address each: 256 tokens at 256 positions 76 us against 73, 512 at 1500 580 against 538).
 //    Positions that only some of the rows see are masked (a later token's value may be anything), the others are not.
-// 32 heads over 8 kv heads, head size 128, 256 tokens at 256 cached positions: 73 us with the append against 800 us with one workgroup per
+// 32 heads over 8 kv heads, head size 128, 256 tokens at 256 cached positions: 70 us with the append against 800 us with one workgroup per
 // (token, head) (attention_kernel), which read the keys and values again for every row and ran each row's chains on one wave.
 // LDS (dynamic): scores [R][scs], 256 floats that reads ahead may touch, key pieces [4][64][16], queries [R][16 ceil(hd/16)].
 template <int R, int RS>
@@ -1270,6 +1272,14 @@ __global__ __launch_bounds__(256) void attention_rows_kernel(const float* __rest
 #pragma unroll
       for (int u = 0; u < 16; ++u) v[u] = vd[(int64_t)min(j0 + u, nmax - 1) * hd];
     };
+    // the same for 16 positions below nmax: one instruction each, the row's offset in a scalar register
+    const uint32_t rowb = (uint32_t)hd * 4u, voff = (uint32_t)min(dim, hd - 1) * 4u;
+    auto load_full = [&](int j0, float (&v)[16]) {
+      const __amdgpu_buffer_rsrc_t rv =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vh) + (int64_t)j0 * hd, (short)0, (int)(16u * rowb), 0x00020000);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, voff, u * rowb, 0));
+    };
 #define ELM_OUT_STEP(n)                                                            \
   _Pragma("unroll") for (int i = 0; i < RPL; ++i) {                                \
     const float pv = row_bcast<n>(p[i]) * v[n];                                    \
@@ -1287,10 +1297,10 @@ __global__ __launch_bounds__(256) void attention_rows_kernel(const float* __rest
     const int nfull = nmin & ~15;  // whole batches that every row sees
     load(0, va);
     int j0 = 0;
-    for (; j0 + 32 <= nfull; j0 += 32) {
-      load(j0 + 16, vb);
+    for (; j0 + 48 <= nfull; j0 += 32) {
+      load_full(j0 + 16, vb);
       batch(j0, va, true);
-      load(j0 + 32, va);
+      load_full(j0 + 32, va);
       batch(j0 + 16, vb, true);
     }
     for (; j0 < nmax; j0 += 16) {
@@ -1333,8 +1343,7 @@ __global__ __launch_bounds__(256) void attention_rows_kernel(const float* __rest
 // every phase that is not one ordered chain is spread over 16 waves:
 //  - scores as in attention_rows_kernel: a lane per position, 64 positions per wave and 1024 per pass, 16 dims of a wave's
 //    key rows at a time through a 4 KB LDS piece of its own, the query broadcast by the multiply;
-//  - the in-order sum of the exponentials on wave 0 while the waves that will add the values request the first 64 positions
-//    and the other waves touch the rest, so that it comes from this XCD's L2 later;
+//  - the in-order sum of the exponentials on wave 0 while the waves that will add the values request the first 64 positions;
 //  - output: a lane per dim, four batches of 16 positions in flight (one position's values are one coalesced request). A wave
 //    that adds issues one instruction in some 5 clocks, so the loop is their count: 3.9 per position with the rows' offsets in
 //    scalar registers against 9.1 with a clamped address each (700 positions 22 -> 17 us, 1900 54 -> 38 us).
@@ -1495,15 +1504,6 @@ __global__ __launch_bounds__(64 * kStepWaves) void attention_step_kernel(
     load(16, v[1]);
     load(32, v[2]);
     load(48, v[3]);
-  } else {
-    // the rest of the value rows into this XCD's L2, one load per 128-byte line
-    const int first = 1 + ((hd + 63) >> 6), step = 64 * (kStepWaves - first) * 32, end = nc * hd;
-    for (int f = 64 * hd + 32 * (64 * (w - first) + lane); f < end; f += 4 * step) {
-      float a[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) a[u] = vh[f + u * step < end ? f + u * step : f];
-      asm volatile("" ::"v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
-    }
   }
   lds_barrier();  // the values stay in flight
   if (!adds) return;
