@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "elm_device_once.h"
+
 namespace elmh {
 
 constexpr int kBlock = 32;       // activation block / q4 group (edgelm kActBlock, kernels.hpp:38)
@@ -163,8 +165,17 @@ hipError_t launch_silu_mul(const float* g, const float* u, float* y, int64_t n, 
 // The non-matmul ops of a layer (elmh_layer.hip), same float order as edgelm's cpu backend.
 hipError_t launch_rmsnorm(const float* x, const float* w, float* y, int rows, int dim, float eps, hipStream_t s);
 // LDS a workgroup may allocate on gfx950 (160 KB per CU; kernels that use more than 64 KB raise their
-// dynamic-LDS limit with hipFuncSetAttribute before the first launch)
+// dynamic-LDS limit before the first launch on each device)
 constexpr size_t kMaxLds = 160 * 1024;
+// The dynamic-LDS limit of `kernel` raised to `bytes` on the current device, at its first call there (once: the kernel's own)
+inline bool raise_dynamic_lds(DeviceOnce& once, const void* kernel, size_t bytes) {
+  int device = 0;
+  const bool ok = hipGetDevice(&device) == hipSuccess && once.run(device, [&] {
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
+  });
+  if (!ok) (void)hipGetLastError();  // the caller takes another kernel or reports it: no later launch does
+  return ok;
+}
 // dynamic LDS the attention kernels may take (their static LDS is a few words; this leaves 1 KB for it)
 constexpr size_t kMaxAttnLds = kMaxLds - 1024;
 size_t attention_lds_bytes(int hd, int n_max);

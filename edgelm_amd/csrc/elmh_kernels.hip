@@ -3230,20 +3230,19 @@ static int64_t gemm_split16_wgs(const GemmArgs& a) {
   for (int i = 0; i < (SW ? 1 : a.n_targets); ++i) rows += (a.tg[i].N + kWave16 - 1) / kWave16;
   return (rows + 7) / 8 * 8 * ((a.T + kWave16 - 1) / kWave16);
 }
+// false: its workgroups don't fit a grid, or their LDS is refused (nothing launched)
 template <int WDT, bool SW, bool TOK>
-static hipError_t gemm_split16_launch(const GemmArgs& a, hipStream_t s) {
-  if (gemm_split16_wgs<SW>(a) > INT32_MAX) return hipErrorInvalidValue;
+static bool gemm_split16_launch(const GemmArgs& a, hipStream_t s) {
+  if (gemm_split16_wgs<SW>(a) > INT32_MAX) return false;
   const int wgs = (int)gemm_split16_wgs<SW>(a);
   auto go = [&](auto gg, auto d) {
     constexpr int G = decltype(gg)::value, D = decltype(d)::value;
     typedef SplitLds<WDT, SW, TOK, G, D> L;
-    if (L::BYTES > 64 * 1024) {
-      static const hipError_t raised = hipFuncSetAttribute((const void*)gemm_split16_kernel<WDT, SW, TOK, G, D>,
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, L::BYTES);
-      if (raised != hipSuccess) return raised;
-    }
+    static DeviceOnce raised;
+    if (L::BYTES > 64 * 1024 && !raise_dynamic_lds(raised, (const void*)gemm_split16_kernel<WDT, SW, TOK, G, D>, L::BYTES))
+      return false;
     gemm_split16_kernel<WDT, SW, TOK, G, D><<<wgs, 64 * L::WAVES, L::BYTES, s>>>(a);
-    return hipGetLastError();
+    return true;
   };
   // one workgroup per CU: longer rounds (q4 4096 x 14336, 16 tokens 22.1 against 23.9 us), or for the per-token sums one more
   // slot (18.6 against 23.7 us); more: two slots of 16 blocks, so that two workgroups fit a CU (64 tokens 57 us; 70 with the
@@ -3267,13 +3266,9 @@ static bool gemm_lds16_launch(const GemmArgs& a, hipStream_t s) {
                              (const void*)gemm_lds16_kernel<WDT, SW, TOK, true, QF, false>,
                              (const void*)gemm_lds16_kernel<WDT, SW, TOK, false, QF, !SW>,
                              (const void*)gemm_lds16_kernel<WDT, SW, TOK, true, QF, !SW>};
-  static bool raised[4] = {false, false, false, false};  // the LDS limit, once per kernel
+  static DeviceOnce raised[4];
   const int which = (mt ? 2 : 0) + (fast ? 1 : 0);
-  if (!raised[which]) {
-    if (hipFuncSetAttribute(ks[which], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds - 1024) != hipSuccess)
-      return false;
-    raised[which] = true;
-  }
+  if (!raise_dynamic_lds(raised[which], ks[which], kMaxLds - 1024)) return false;
   constexpr int RW = QF ? 32 : 16, TW = QF ? 32 : 64;
   int rows = 0;
   for (int i = 0; i < (SW ? 1 : a.n_targets); ++i) rows += (a.tg[i].N + RW - 1) / RW;
@@ -3355,7 +3350,7 @@ static hipError_t gemm_go(const GemmArgs& a, int tiles, hipStream_t s) {
   const char* const forced = getenv("ELMH_GEMM_KERNEL");
   const bool split = forced ? std::strcmp(forced, "split") == 0
                             : a.nb > kLds16MaxBlocks && split_wgs <= (SW ? 1200 : 2048) && !getenv("ELMH_GEMM_TOKEN_TILE");
-  if (split && !a.fast && a.H >= 4 && !(a.H & (a.H - 1))) return gemm_split16_launch<WDT, SW, TOK>(a, s);
+  if (split && !a.fast && a.H >= 4 && !(a.H & (a.H - 1)) && gemm_split16_launch<WDT, SW, TOK>(a, s)) return hipGetLastError();
   if (wave) {
     if (wave32)
       gemm_wave_launch<WDT, SW, TOK>(a, s);
@@ -3441,13 +3436,9 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
     b.tile_start[n] = tiles;
     const size_t lds = f32q4_lds_bytes(a.K, a.nb, rt, nsel, a.nw != nullptr);
     if (tiles < 1) return hipErrorInvalidValue;
-    static bool raised[2] = {false, false};  // the LDS limit, once per kernel
-    if (lds > 64 * 1024 && !raised[nsel - 1]) {
-      const void* k = swiglu ? (const void*)gemv_f32act_q4_kernel<true> : (const void*)gemv_f32act_q4_kernel<false>;
-      const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds - 1024);
-      if (e != hipSuccess) return e;
-      raised[nsel - 1] = true;
-    }
+    static DeviceOnce raised[2];
+    const void* const k = swiglu ? (const void*)gemv_f32act_q4_kernel<true> : (const void*)gemv_f32act_q4_kernel<false>;
+    if (lds > 64 * 1024 && !raise_dynamic_lds(raised[nsel - 1], k, kMaxLds - 1024)) return hipErrorInvalidValue;
     if (swiglu) gemv_f32act_q4_kernel<true><<<tiles, 256, lds, s>>>(b);
     else gemv_f32act_q4_kernel<false><<<tiles, 256, lds, s>>>(b);
     return hipGetLastError();

@@ -1892,7 +1892,8 @@ static size_t attention_step_lds_bytes(int hd, int n_cap) {
   return ((size_t)((n_cap + 15) & ~15) + 256 + kStepWaves * 1024 + 2 * (size_t)((hd + 15) & ~15)) * sizeof(float);
 }
 
-// the attention kernels keep a whole score row (and a chunk of values) in LDS: allow them up to kMaxAttnLds
+// the attention kernels keep a whole score row (and a chunk of values) in LDS: allow them up to kMaxAttnLds on the current
+// device
 bool raise_lds_limit() {
   const void* kernels[] = {(const void*)attention_kernel<64, false>, (const void*)attention_kernel<0, false>,
                            (const void*)attention_kernel<64, true>, (const void*)attention_kernel<0, true>,
@@ -1948,8 +1949,9 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, floa
   }
   const float* kn = fuse ? k : nullptr;
   const float* vn = fuse ? v : nullptr;
-  static const bool lds_ok = raise_lds_limit();  // once per process (the attribute holds for the kernel)
-  if (!lds_ok) return hipErrorInvalidValue;
+  static DeviceOnce raised;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || !raised.run(device, raise_lds_limit)) return hipErrorInvalidValue;
   if (step) {
     const dim3 grid(n_kv, grp, T);
     const size_t lds = attention_step_lds_bytes(hd, n_cap);
