@@ -1,0 +1,107 @@
+// Which kernel a call takes, where that depends on sizes, types and alignment: the rules alone, in plain C++ (no HIP), so
+// that they can be checked without a GPU. The launchers ask here; each rule's comment says what both sides measured.
+#pragma once
+#include <cstddef>
+#include <cstdint>
+
+namespace elmh {
+
+// LDS a workgroup may allocate on gfx950 (160 KB per CU; kernels that use more than 64 KB raise their
+// dynamic-LDS limit before the first launch on each device)
+constexpr size_t kMaxLds = 160 * 1024;
+// dynamic LDS the attention kernels may take (their static LDS is a few words; this leaves 1 KB for it)
+constexpr size_t kMaxAttnLds = kMaxLds - 1024;
+
+// ---------------------------------------------------------------- attention
+
+constexpr int kAttnThreads = 256;
+constexpr int kAttnVF = 20;                           // attention_kernel: float4 of values per thread per chunk
+constexpr int kAttnChunkF4 = kAttnThreads * kAttnVF;  // 80 KB: 320 positions of head size 64
+constexpr int attn_chunk_pos(int hd) { return (kAttnChunkF4 / (hd / 4)) & ~15; }
+constexpr int kDecRows = 256;    // attention_decode64_kernel: rows per LDS buffer, one per thread
+constexpr int kAttnQ = 4;        // attention_prefill_kernel, attention_prefill64_kernel: query tokens per workgroup
+constexpr int kAttnPVPos = 96;   // attention_prefill_kernel: value rows per chunk (24 KB)
+constexpr int kPfRows = 128;     // attention_prefill64_kernel: key and value rows per LDS chunk
+constexpr int kStepWaves = 16;   // attention_step_kernel
+
+// LDS of each kernel for n_cap score slots
+inline size_t attention_decode_lds_bytes(int n_cap) {  // two row buffers, the scores, q and the step's key
+  return ((size_t)2 * kDecRows * 64 + (size_t)((n_cap + 255) & ~255) + 128) * sizeof(float);
+}
+inline size_t attention_prefill_lds_bytes(int n_cap) {
+  return ((size_t)kAttnQ * 64 + (size_t)kAttnQ * ((n_cap + 63) & ~63) + (size_t)kAttnPVPos * 64) * sizeof(float);
+}
+inline size_t attention_prefill64_lds_bytes(int n_cap) {
+  return ((size_t)2 * kPfRows * 64 + (size_t)kAttnQ * ((n_cap + 255) & ~255) + (size_t)kAttnQ * 64) * sizeof(float);
+}
+inline size_t attention_lds_bytes(int hd, int n_max) {
+  const size_t hdp = (size_t)((hd + 3) & ~3);
+  return (2 * hdp + (size_t)((n_max + 63) & ~63) + (size_t)attn_chunk_pos(hd) * hd) * sizeof(float);
+}
+// attention_kernel with its score rows in global memory: LDS holds q, the fused key and a chunk
+inline size_t attention_gs_lds_bytes(int hd) {
+  return (2 * (size_t)((hd + 3) & ~3) + (size_t)attn_chunk_pos(hd) * hd) * sizeof(float);
+}
+// attention_rows_kernel for R rows per workgroup: the score row stride (a multiple of 4 that spreads the rows over the LDS
+// banks) and the LDS it takes
+inline int attention_rows_stride(int n_cap) { return ((n_cap + 63) & ~63) + 20; }
+inline size_t attention_rows_lds_bytes(int R, int hd, int n_cap) {
+  return ((size_t)R * attention_rows_stride(n_cap) + 256 + 4 * 1024 + (size_t)R * ((hd + 15) & ~15)) * sizeof(float);
+}
+inline size_t attention_step_lds_bytes(int hd, int n_cap) {
+  return ((size_t)((n_cap + 15) & ~15) + 256 + kStepWaves * 1024 + 2 * (size_t)((hd + 15) & ~15)) * sizeof(float);
+}
+
+enum class AttnKernel {
+  kStep,       // attention_step_kernel: a workgroup per (token, head)
+  kRows4,      // attention_rows_kernel, 4 rows a workgroup
+  kRows8,      //   and 8
+  kPrefill64,  // attention_prefill64_kernel (the append inside)
+  kPrefill,    // attention_prefill_kernel
+  kDecode64,   // attention_decode64_kernel
+  kWhole,      // attention_kernel, its score row in LDS
+  kGlobal,     // attention_kernel, its score rows in global memory
+};
+
+struct AttnCall {
+  int T;         // query tokens
+  int n_cap;     // score slots: pos0 + T, or with the position in device memory the whole cache
+  bool pos_dev;  // the position is in device memory (T == 1)
+  int n_heads, n_kv, hd;
+  bool quant;     // the output is asked for as the next GEMM's operand too (T > 1, head size 64)
+  bool aligned;   // the key cache starts on 16 bytes
+};
+
+inline AttnKernel attention_route(const AttnCall& c) {
+  const bool fuse = c.T == 1;
+  const int grp = c.n_heads / c.n_kv;
+  const int64_t pairs = (int64_t)c.T * c.n_heads;
+  // The step and rows kernels copy key rows to LDS 16 bytes at a time; a key cache that starts elsewhere takes the kernels
+  // that load them into registers (at head size 64 those that it took before: they copy rows too, except attention_kernel).
+  //
+  // A chunk of at most one (token, head) per CU: a 1024-thread workgroup each (32 heads of size 128 over 1000 cached
+  // positions: 35 / 38 us for 2 / 8 tokens, against 51 us with rows of four in 256-thread workgroups; 16 tokens 55 against
+  // 52). At head size 64 only where no GEMM operand is asked for (8 tokens of 9 heads over 300 positions: 13.7 against 17.9
+  // us with attention_prefill64_kernel). One token: always, but for the head-size-64 kernel's caches (it takes the step's
+  // rows before it knows the position: 6.0 against 8.6 us at 200 positions, 15.4 against 19.9 at 700).
+  const bool step_fits = c.aligned && grp < 65536 && attention_step_lds_bytes(c.hd, c.n_cap) <= kMaxAttnLds;
+  const bool step = step_fits && (fuse ? c.hd != 64 || attention_decode_lds_bytes(c.n_cap) > kMaxAttnLds
+                                       : !c.pos_dev && pairs <= 256 && (c.hd != 64 || !c.quant));
+  if (step) return AttnKernel::kStep;
+  // Longer chunks: attention_rows_kernel, at head size 64 from 4096 (token, head) pairs on (9 heads: 512 tokens 31 against
+  // 48 us with attention_prefill64_kernel, 128 tokens 11 against 8.4; 32 heads, 64 tokens at 600 positions 34 against 32).
+  // R = 8 rows a workgroup read the keys half as often as 4; 4 fill the chip at fewer rows and keep more workgroups per CU
+  // where the score rows are long (32 heads of size 128: 256 tokens at 256 positions 80 against 86 us; 128 tokens 19.5
+  // against 17.4; 512 at 1500 986 against 613).
+  auto groups = [&](int R) { return ((int64_t)c.T * grp + R - 1) / R; };
+  const int R = c.n_kv * groups(8) >= 1024 && 3 * attention_rows_lds_bytes(8, c.hd, c.n_cap) <= kMaxLds ? 8 : 4;
+  if (!fuse && !c.pos_dev && c.aligned && groups(R) < 65536 && (c.hd != 64 || pairs >= 4096) &&
+      attention_rows_lds_bytes(R, c.hd, c.n_cap) <= kMaxAttnLds)
+    return R == 8 ? AttnKernel::kRows8 : AttnKernel::kRows4;
+  if (!fuse && c.hd == 64 && !c.pos_dev && attention_prefill64_lds_bytes(c.n_cap) <= kMaxAttnLds) return AttnKernel::kPrefill64;
+  if (!fuse && c.hd == 64 && attention_prefill_lds_bytes(c.n_cap) <= kMaxAttnLds) return AttnKernel::kPrefill;
+  if (fuse && c.hd == 64 && attention_decode_lds_bytes(c.n_cap) <= kMaxAttnLds) return AttnKernel::kDecode64;
+  return attention_lds_bytes(c.hd, c.n_cap) <= kMaxAttnLds ? AttnKernel::kWhole : AttnKernel::kGlobal;
+}
+
+}  // namespace elmh

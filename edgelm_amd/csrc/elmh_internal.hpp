@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "elm_device_once.h"
+#include "elm_routes.h"
 
 namespace elmh {
 
@@ -164,9 +165,6 @@ bool f32act_q4_ok(int T, int K, int nb, int H, int nsel, int rows, bool norm);
 hipError_t launch_silu_mul(const float* g, const float* u, float* y, int64_t n, hipStream_t s);
 // The non-matmul ops of a layer (elmh_layer.hip), same float order as edgelm's cpu backend.
 hipError_t launch_rmsnorm(const float* x, const float* w, float* y, int rows, int dim, float eps, hipStream_t s);
-// LDS a workgroup may allocate on gfx950 (160 KB per CU; kernels that use more than 64 KB raise their
-// dynamic-LDS limit before the first launch on each device)
-constexpr size_t kMaxLds = 160 * 1024;
 // The dynamic-LDS limit of `kernel` raised to `bytes` on the current device, at its first call there (once: the kernel's own)
 inline bool raise_dynamic_lds(DeviceOnce& once, const void* kernel, size_t bytes) {
   int device = 0;
@@ -176,9 +174,6 @@ inline bool raise_dynamic_lds(DeviceOnce& once, const void* kernel, size_t bytes
   if (!ok) (void)hipGetLastError();  // the caller takes another kernel or reports it: no later launch does
   return ok;
 }
-// dynamic LDS the attention kernels may take (their static LDS is a few words; this leaves 1 KB for it)
-constexpr size_t kMaxAttnLds = kMaxLds - 1024;
-size_t attention_lds_bytes(int hd, int n_max);
 // Bytes of global score rows launch_attention needs for this call (0: the rows fit LDS). pos_dev: the
 // position comes from device memory (rows sized for max_ctx).
 size_t attention_global_score_bytes(int T, int pos0, bool pos_dev, int n_heads, int hd, int max_ctx);

@@ -170,11 +170,6 @@ __global__ __launch_bounds__(64) void kv_append_kernel(const float* __restrict__
 // rounded up to 64 floats per workgroup) and LDS keeps q and the product chunk only; the in-order sum
 // of the exponentials then passes them through the product region a chunk at a time. Same float
 // operations in the same order.
-constexpr int kAttnThreads = 256;
-constexpr int kAttnVF = 20;                           // float4 of values per thread per chunk
-constexpr int kAttnChunkF4 = kAttnThreads * kAttnVF;  // 80 KB: 320 positions of head size 64
-
-__device__ __host__ __forceinline__ int attn_chunk_pos(int hd) { return (kAttnChunkF4 / (hd / 4)) & ~15; }
 
 __device__ __forceinline__ float dot_row(const float* __restrict__ q, const float* __restrict__ k, int hd) {
   if (hd == 64) {  // the common head size: all 16 loads issued before the first product
@@ -467,7 +462,6 @@ __global__ __launch_bounds__(kAttnThreads) void attention_kernel(const float* __
 // buffer, values alternating between both, the next chunk in flight while wave 0 adds the current.
 // LDS (dynamic): keys [C][64], values [C][64], scores [n_cap rounded up to 256], q [64], the
 // step's rotated key [64].
-constexpr int kDecRows = 256;  // C: rows per LDS buffer, one per thread
 
 // dot_f32_scalar's order (four strided accumulators, then (s0 + s1) + (s2 + s3)) of q and a row
 // in LDS whose chunk u sits in slot u ^ swz
@@ -714,9 +708,6 @@ __global__ __launch_bounds__(256) void attention_decode64_kernel(
 // attention_kernel (cpu::attention): scores by dot_f32_scalar's order, max, expf(s - max), the sum
 // in increasing position, p_j = e_j * inv, o_i += p_j * v_j[i] in increasing position.
 // LDS (dynamic): q [kAttnQ][64], scores [kAttnQ][n_cap rounded up to 64], values [kAttnPVPos][64].
-constexpr int kAttnQ = 4;
-constexpr int kAttnPVPos = 96;  // value rows per chunk (24 KB)
-
 __global__ __launch_bounds__(256) void attention_prefill_kernel(const float* __restrict__ q, float* __restrict__ out,
                                                                 const float* __restrict__ kc,
                                                                 const float* __restrict__ vc, int pos0, int T,
@@ -868,8 +859,6 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(const float* __r
 // launch reads them there).
 // LDS (dynamic): keys [kPfRows][64] (chunk u of row r in slot u ^ (r & 15)), values [kPfRows][64],
 // scores [kAttnQ][n_cap rounded up to 256], q [kAttnQ][64].
-constexpr int kPfRows = 128;
-
 __global__ __launch_bounds__(256) void attention_prefill64_kernel(
     const float* __restrict__ q, float* __restrict__ out, float* __restrict__ kc, float* __restrict__ vc, int pos0,
     int T, int grp, int n_kv, int max_ctx, int n_cap, const float* __restrict__ rcos, const float* __restrict__ rsin,
@@ -1352,7 +1341,6 @@ __global__ __launch_bounds__(256) void attention_rows_kernel(const float* __rest
 // 32 heads over 8 kv heads, head size 128, 700 cached positions: 17 us against 44 us with attention_kernel.
 // LDS (dynamic): scores [n_cap rounded up to 16, and 256 more that reads ahead may touch], key pieces [16][64][16], query and
 // step's key [16 ceil(hd / 16)] each.
-constexpr int kStepWaves = 16;
 template <bool FUSE>
 __global__ __launch_bounds__(64 * kStepWaves) void attention_step_kernel(
     const float* __restrict__ q, float* __restrict__ out, float* __restrict__ kc, float* __restrict__ vc, int pos0,
@@ -1847,49 +1835,24 @@ hipError_t launch_rmsnorm(const float* x, const float* w, float* y, int rows, in
   return hipGetLastError();
 }
 
-// attention_decode64_kernel: two row buffers, the scores (a multiple of 256), q and the step's key
-size_t attention_decode_lds_bytes(int n_cap) {
-  return ((size_t)2 * kDecRows * 64 + (size_t)((n_cap + 255) & ~255) + 128) * sizeof(float);
-}
-
-size_t attention_lds_bytes(int hd, int n_max) {
-  const size_t hdp = (size_t)((hd + 3) & ~3);
-  return (2 * hdp + (size_t)((n_max + 63) & ~63) + (size_t)attn_chunk_pos(hd) * hd) * sizeof(float);
-}
-
-// attention_kernel with its score rows in global memory (GS): LDS holds q, the fused key and a chunk
-static size_t attention_gs_lds_bytes(int hd) {
-  return (2 * (size_t)((hd + 3) & ~3) + (size_t)attn_chunk_pos(hd) * hd) * sizeof(float);
-}
-
 size_t attention_global_score_bytes(int T, int pos0, bool pos_dev, int n_heads, int hd, int max_ctx) {
   const int n_cap = pos_dev ? max_ctx : pos0 + T;
   if (attention_lds_bytes(hd, n_cap) <= kMaxAttnLds) return 0;
   return (size_t)T * n_heads * (size_t)((n_cap + 63) & ~63) * sizeof(float);
 }
 
-// attention_rows_kernel for R rows per workgroup: the score row stride (a multiple of 4 that spreads the rows over the LDS
-// banks) and the LDS it takes
-static int attn_rows_stride(int n_cap) { return ((n_cap + 63) & ~63) + 20; }
-static size_t attention_rows_lds_bytes(int R, int hd, int n_cap) {
-  return ((size_t)R * attn_rows_stride(n_cap) + 256 + 4 * 1024 + (size_t)R * ((hd + 15) & ~15)) * sizeof(float);
-}
 template <int R>
 static hipError_t launch_attention_rows(const float* q, float* out, const float* kc, const float* vc, int T, int pos0, int grp,
                                         int n_kv, int hd, int max_ctx, const float* rcos, const float* rsin, int8_t* xq,
                                         float* xd, int Tpad, hipStream_t s) {
   const dim3 grid(n_kv, (T * grp + R - 1) / R);
   const size_t lds = attention_rows_lds_bytes(R, hd, pos0 + T);
-  const int scs = attn_rows_stride(pos0 + T);
+  const int scs = attention_rows_stride(pos0 + T);
   if (hd <= 64)
     attention_rows_kernel<R, 2><<<grid, 256, lds, s>>>(q, out, kc, vc, pos0, T, grp, n_kv, hd, max_ctx, scs, rcos, rsin, xq, xd, Tpad);
   else
     attention_rows_kernel<R, 1><<<grid, 256, lds, s>>>(q, out, kc, vc, pos0, T, grp, n_kv, hd, max_ctx, scs, rcos, rsin, xq, xd, Tpad);
   return hipGetLastError();
-}
-
-static size_t attention_step_lds_bytes(int hd, int n_cap) {
-  return ((size_t)((n_cap + 15) & ~15) + 256 + kStepWaves * 1024 + 2 * (size_t)((hd + 15) & ~15)) * sizeof(float);
 }
 
 // the attention kernels keep a whole score row (and a chunk of values) in LDS: allow them up to kMaxAttnLds on the current
@@ -1910,6 +1873,8 @@ bool raise_lds_limit() {
   return true;
 }
 
+static bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
 hipError_t launch_attention(const float* q, const float* k, const float* v, float* out, int T, int pos0,
                             const int* pos_dev, int n_heads, int n_kv, int hd, float* kc, float* vc, int max_ctx,
                             const float* rcos, const float* rsin, hipStream_t s, int8_t* xq, float* xd, int Tpad,
@@ -1917,32 +1882,13 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, floa
   if (quantized) *quantized = false;
   // with the position in device memory the score buffer covers the whole cache
   const int n_cap = pos_dev ? max_ctx : pos0 + T;  // score slots
+  const int grp = n_heads / n_kv;
+  const bool quant = xq && xd && quantized;
+  const AttnKernel route = attention_route({T, n_cap, pos_dev != nullptr, n_heads, n_kv, hd, quant, aligned16(kc)});
   // one token, and chunks on the head-size-64 prefill kernel: the append runs inside the attention
   // kernel; other chunks append every key first
   const bool fuse = T == 1;
-  const int grp = n_heads / n_kv;
-  const bool quant = xq && xd && quantized;
-  const size_t lds_pf = ((size_t)kAttnQ * hd + (size_t)kAttnQ * ((n_cap + 63) & ~63) + (size_t)kAttnPVPos * hd) * 4;
-  const size_t lds_pf64 = ((size_t)2 * kPfRows * 64 + (size_t)kAttnQ * ((n_cap + 255) & ~255) + (size_t)kAttnQ * 64) * 4;
-  // A chunk of at most one (token, head) per CU: a 1024-thread workgroup each (32 heads of size 128 over 1000 cached
-  // positions: 35 / 38 us for 2 / 8 tokens, against 51 us with rows of four in 256-thread workgroups; 16 tokens 55 against
-  // 52). At head size 64 only where no GEMM operand is asked for (8 tokens of 9 heads over 300 positions: 13.7 against 17.9
-  // us with attention_prefill64_kernel). One token: always, but for the head-size-64 kernel's caches (it takes the step's
-  // rows before it knows the position: 6.0 against 8.6 us at 200 positions, 15.4 against 19.9 at 700).
-  const bool step_fits = attention_step_lds_bytes(hd, n_cap) <= kMaxAttnLds;
-  const bool step = step_fits && (fuse ? hd != 64 || attention_decode_lds_bytes(n_cap) > kMaxAttnLds
-                                       : !pos_dev && (int64_t)T * n_heads <= 256 && (hd != 64 || !quant));
-  // Longer chunks: attention_rows_kernel, at head size 64 from 4096 (token, head) pairs on (9 heads: 512 tokens 31 against
-  // 48 us with attention_prefill64_kernel, 128 tokens 11 against 8.4; 32 heads, 64 tokens at 600 positions 34 against 32).
-  // R = 8 rows a workgroup read the keys half as often as 4; 4 fill the chip at fewer rows and keep more workgroups per CU
-  // where the score rows are long (32 heads of size 128: 256 tokens at 256 positions 80 against 86 us; 128 tokens 19.5
-  // against 17.4; 512 at 1500 986 against 613).
-  auto wgs = [&](int R) { return (int64_t)n_kv * (((int64_t)T * grp + R - 1) / R); };
-  const int R = wgs(8) >= 1024 && 3 * attention_rows_lds_bytes(8, hd, n_cap) <= kMaxLds ? 8 : 4;
-  const bool rows = !fuse && !pos_dev && !step && wgs(R) / n_kv < 65536 && (hd != 64 || (int64_t)T * n_heads >= 4096) &&
-                    attention_rows_lds_bytes(R, hd, n_cap) <= kMaxAttnLds;
-  const bool pf64 = !fuse && hd == 64 && lds_pf64 <= kMaxAttnLds && !pos_dev && !step && !rows;
-  if (!fuse && !pf64) {
+  if (!fuse && route != AttnKernel::kPrefill64) {
     kv_append_kernel<<<T * n_kv, 64, 0, s>>>(k, v, kc, vc, pos0, pos_dev, n_kv, hd, max_ctx, rcos, rsin);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1952,7 +1898,7 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, floa
   static DeviceOnce raised;
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || !raised.run(device, raise_lds_limit)) return hipErrorInvalidValue;
-  if (step) {
+  if (route == AttnKernel::kStep) {
     const dim3 grid(n_kv, grp, T);
     const size_t lds = attention_step_lds_bytes(hd, n_cap);
     if (fuse)
@@ -1963,43 +1909,42 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, floa
                                                                       n_cap, rcos, rsin, nullptr, nullptr);
     return hipGetLastError();
   }
-  if (rows) {
-    const hipError_t e = R == 8 ? launch_attention_rows<8>(q, out, kc, vc, T, pos0, grp, n_kv, hd, max_ctx, rcos, rsin, quant ? xq : nullptr, xd, Tpad, s)
-                                : launch_attention_rows<4>(q, out, kc, vc, T, pos0, grp, n_kv, hd, max_ctx, rcos, rsin, quant ? xq : nullptr, xd, Tpad, s);
+  if (route == AttnKernel::kRows8 || route == AttnKernel::kRows4) {
+    const auto launch = route == AttnKernel::kRows8 ? launch_attention_rows<8> : launch_attention_rows<4>;
+    const hipError_t e = launch(q, out, kc, vc, T, pos0, grp, n_kv, hd, max_ctx, rcos, rsin, quant ? xq : nullptr, xd, Tpad, s);
     if (e == hipSuccess && quant) *quantized = true;
     return e;
   }
-  if (pf64) {
+  if (route == AttnKernel::kPrefill64) {
     const int ngr = (T + kAttnQ - 1) / kAttnQ;
-    attention_prefill64_kernel<<<dim3(ngr, n_heads / n_kv, n_kv), 256, lds_pf64, s>>>(
-        q, out, kc, vc, pos0, T, n_heads / n_kv, n_kv, max_ctx, n_cap, rcos, rsin, quant ? xq : nullptr,
+    attention_prefill64_kernel<<<dim3(ngr, grp, n_kv), 256, attention_prefill64_lds_bytes(n_cap), s>>>(
+        q, out, kc, vc, pos0, T, grp, n_kv, max_ctx, n_cap, rcos, rsin, quant ? xq : nullptr,
         quant ? xd : nullptr, Tpad, k, v);
     const hipError_t e = hipGetLastError();
     if (e == hipSuccess && quant) *quantized = true;
     return e;
   }
-  if (!fuse && hd == 64 && lds_pf <= kMaxAttnLds) {
+  if (route == AttnKernel::kPrefill) {
     const int ngr = (T + kAttnQ - 1) / kAttnQ;
-    attention_prefill_kernel<<<n_heads * ngr, 256, lds_pf, s>>>(q, out, kc, vc, pos0, T, n_heads, n_kv, max_ctx, n_cap,
-                                                                rcos, rsin, quant ? xq : nullptr,
-                                                                quant ? xd : nullptr, Tpad);
+    attention_prefill_kernel<<<n_heads * ngr, 256, attention_prefill_lds_bytes(n_cap), s>>>(
+        q, out, kc, vc, pos0, T, n_heads, n_kv, max_ctx, n_cap, rcos, rsin, quant ? xq : nullptr, quant ? xd : nullptr, Tpad);
     const hipError_t e = hipGetLastError();
     if (e == hipSuccess && quant) *quantized = true;
     return e;
   }
-  const bool in_lds = attention_lds_bytes(hd, n_cap) <= kMaxAttnLds;
-  if (!in_lds && !gscores) return hipErrorInvalidValue;  // a score row past LDS needs the global rows
+  if (route == AttnKernel::kGlobal && !gscores) return hipErrorInvalidValue;  // a score row past LDS needs the global rows
+  // attention_kernel, one token with the append inside (where its row fits LDS: only from a key cache off 16 bytes)
   const size_t lds_gs = attention_gs_lds_bytes(hd), lds = attention_lds_bytes(hd, n_cap);
-  if (fuse && hd == 64 && attention_decode_lds_bytes(n_cap) <= kMaxAttnLds)
-    attention_decode64_kernel<<<dim3(n_kv, n_heads / n_kv), 256, attention_decode_lds_bytes(n_cap), s>>>(
-        q, out, kc, vc, pos0, pos_dev, n_heads / n_kv, n_kv, max_ctx, n_cap, rcos, rsin, k, v);
-  else if (hd == 64 && in_lds)
+  if (route == AttnKernel::kDecode64)
+    attention_decode64_kernel<<<dim3(n_kv, grp), 256, attention_decode_lds_bytes(n_cap), s>>>(
+        q, out, kc, vc, pos0, pos_dev, grp, n_kv, max_ctx, n_cap, rcos, rsin, k, v);
+  else if (hd == 64 && route == AttnKernel::kWhole)
     attention_kernel<64, false><<<T * n_heads, kAttnThreads, lds, s>>>(
         q, out, kc, vc, pos0, pos_dev, n_heads, n_kv, hd, max_ctx, n_cap, rcos, rsin, kn, vn, nullptr);
   else if (hd == 64)
     attention_kernel<64, true><<<T * n_heads, kAttnThreads, lds_gs, s>>>(
         q, out, kc, vc, pos0, pos_dev, n_heads, n_kv, hd, max_ctx, n_cap, rcos, rsin, kn, vn, gscores);
-  else if (in_lds)
+  else if (route == AttnKernel::kWhole)
     attention_kernel<0, false><<<T * n_heads, kAttnThreads, lds, s>>>(
         q, out, kc, vc, pos0, pos_dev, n_heads, n_kv, hd, max_ctx, n_cap, rcos, rsin, kn, vn, nullptr);
   else

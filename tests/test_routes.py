@@ -1,0 +1,41 @@
+"""elm_routes.h, the rules that pick a kernel by sizes, types and alignment, compiled by the host compiler and asked without a
+GPU: each rule at the calls that were measured on both of its sides, and over the forms that it accepts."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SHIM = r"""
+#include "elm_routes.h"
+using namespace elmh;
+extern "C" int attn(int T, int n_cap, int pos_dev, int nh, int nkv, int hd, int quant, int aligned) {
+  return (int)attention_route({T, n_cap, pos_dev != 0, nh, nkv, hd, quant != 0, aligned != 0});
+}
+"""
+STEP, ROWS4, ROWS8, PREFILL64, PREFILL, DECODE64, WHOLE, GLOBAL = range(8)
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory):
+    d = tmp_path_factory.mktemp("routes")
+    (d / "shim.cpp").write_text(SHIM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I",
+                    os.path.join(ROOT, "edgelm_amd", "csrc"), str(d / "shim.cpp"), "-o", str(d / "routes.so")], check=True)
+    return C.CDLL(str(d / "routes.so"))
+
+
+def test_attention_key_cache_off_16_bytes(routes):
+    """The kernels that copy key rows to LDS 16 bytes at a time take no key cache that starts elsewhere: head sizes other
+    than 64 go to attention_kernel, 64 to the kernels that it has of its own."""
+    for T in (1, 2, 7, 33, 300, 2048):
+        for nh, nkv in ((1, 1), (9, 3), (32, 8), (32, 32)):
+            for n in (T, 300 + T, 9500 + T, 23000 + T, 40000 + T):
+                for hd in (4, 20, 80, 128, 256):
+                    assert routes.attn(T, n, 0, nh, nkv, hd, 0, 0) in (WHOLE, GLOBAL)
+                assert routes.attn(T, n, 0, nh, nkv, 64, 0, 0) not in (STEP, ROWS4, ROWS8)
+    assert routes.attn(1, 2048, 1, 32, 8, 128, 0, 0) == WHOLE
+    assert routes.attn(1, 2048, 1, 32, 8, 128, 0, 1) == STEP
+    assert routes.attn(256, 512, 0, 32, 8, 128, 0, 1) == ROWS8
