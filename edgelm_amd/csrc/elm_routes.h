@@ -104,4 +104,10 @@ inline AttnKernel attention_route(const AttnCall& c) {
   return attention_lds_bytes(c.hd, c.n_cap) <= kMaxAttnLds ? AttnKernel::kWhole : AttnKernel::kGlobal;
 }
 
+// Bytes of global score rows the call needs (0 unless it takes attention_kernel with its score rows in global memory)
+inline size_t attention_global_score_bytes(const AttnCall& c) {
+  if (attention_route(c) != AttnKernel::kGlobal) return 0;
+  return (size_t)c.T * c.n_heads * (size_t)((c.n_cap + 63) & ~63) * sizeof(float);
+}
+
 }  // namespace elmh

@@ -656,9 +656,9 @@ int check_attention(elmh_ctx* c, const float* q, const float* k, const float* v,
   return ELMH_OK;
 }
 
-// The global score rows of an attention call whose rows do not fit LDS (null when they do).
-int attention_scores(elmh_ctx* c, int T, int pos0, bool pos_dev, int n_heads, int head_dim, int max_ctx, float** out) {
-  const size_t bytes = attention_global_score_bytes(T, pos0, pos_dev, n_heads, head_dim, max_ctx);
+// The global score rows of an attention call that keeps them there (null for the others).
+int attention_scores(elmh_ctx* c, const AttnCall& call, float** out) {
+  const size_t bytes = attention_global_score_bytes(call);
   *out = nullptr;
   if (!bytes) return ELMH_OK;
   if (const int rc = ensure(c, c->asc, bytes)) return rc;
@@ -1295,7 +1295,8 @@ int elmh_attention_matmul_dev(elmh_ctx* c, const float* q, const float* k, const
   bool quantized = false;
   c->attn_fused = 0;
   float* gsc = nullptr;
-  if ((rc = attention_scores(c, T, pos0, false, n_heads, head_dim, max_ctx, &gsc))) return rc;
+  if ((rc = attention_scores(c, attention_call(T, pos0, false, n_heads, n_kv, head_dim, k_cache, max_ctx, xq != nullptr), &gsc)))
+    return rc;
   HIP_OR_FAIL(c, launch_attention(q, k, v, out, T, pos0, nullptr, n_heads, n_kv, head_dim, k_cache, v_cache, max_ctx,
                                   rope_cos, rope_sin, c->stream, xq, xd, Tpad, &quantized, gsc));
   c->attn_fused = quantized ? 1 : 0;
@@ -1315,7 +1316,8 @@ int elmh_attention_dev(elmh_ctx* c, const float* q, const float* k, const float*
   if (rc) return rc;
   DeviceGuard g(c);
   float* gsc = nullptr;
-  if (const int r2 = attention_scores(c, T, pos0, false, n_heads, head_dim, max_ctx, &gsc)) return r2;
+  if (const int r2 = attention_scores(c, attention_call(T, pos0, false, n_heads, n_kv, head_dim, k_cache, max_ctx, false), &gsc))
+    return r2;
   HIP_OR_FAIL(c, launch_attention(q, k, v, out, T, pos0, nullptr, n_heads, n_kv, head_dim, k_cache, v_cache, max_ctx,
                                   rope_cos, rope_sin, c->stream, nullptr, nullptr, 0, nullptr, gsc));
   return ELMH_OK;
@@ -1336,7 +1338,8 @@ int elmh_attention_step_dev(elmh_ctx* c, const float* q, const float* k, const f
   if (!rope_cos != !rope_sin) return fail(c, ELMH_ERR_ARG, "attention_step: rope_cos and rope_sin go together");
   DeviceGuard g(c);
   float* gsc = nullptr;
-  if (const int rc = attention_scores(c, 1, 0, true, n_heads, head_dim, max_ctx, &gsc)) return rc;
+  if (const int rc = attention_scores(c, attention_call(1, 0, true, n_heads, n_kv, head_dim, k_cache, max_ctx, false), &gsc))
+    return rc;
   HIP_OR_FAIL(c, launch_attention(q, k, v, out, 1, 0, pos_dev, n_heads, n_kv, head_dim, k_cache, v_cache, max_ctx,
                                   rope_cos, rope_sin, c->stream, nullptr, nullptr, 0, nullptr, gsc));
   return ELMH_OK;

@@ -174,16 +174,19 @@ inline bool raise_dynamic_lds(DeviceOnce& once, const void* kernel, size_t bytes
   if (!ok) (void)hipGetLastError();  // the caller takes another kernel or reports it: no later launch does
   return ok;
 }
-// Bytes of global score rows launch_attention needs for this call (0: the rows fit LDS). pos_dev: the
-// position comes from device memory (rows sized for max_ctx).
-size_t attention_global_score_bytes(int T, int pos0, bool pos_dev, int n_heads, int hd, int max_ctx);
+// The call as attention_route and attention_global_score_bytes take it. pos_dev: the position comes from device memory (the
+// scores are sized for max_ctx); quant: xq, xd and quantized are given.
+inline AttnCall attention_call(int T, int pos0, bool pos_dev, int n_heads, int n_kv, int hd, const float* kc, int max_ctx,
+                               bool quant) {
+  return {T, pos_dev ? max_ctx : pos0 + T, pos_dev, n_heads, n_kv, hd, quant, reinterpret_cast<uintptr_t>(kc) % 16 == 0};
+}
 // pos_dev (if not null): pos0 read from device memory (T must be 1; LDS sized for max_ctx).
 // xq, xd, Tpad, quantized (all given): where the chunk kernel (T > 1, head size 64) runs, it also
 // writes its output as the block-scale GEMM's activation fragments (xq, Tpad * n_heads * hd bytes)
 // and scales (xd, 2 * n_heads * Tpad floats; tokens T .. Tpad-1 left as they were) and sets
 // *quantized; otherwise *quantized is false and xq, xd are untouched.
 // gscores: attention_global_score_bytes() of device memory where that is not 0 (score rows longer than
-// LDS holds); without it such a call fails with hipErrorInvalidValue.
+// LDS holds, on the kernel that takes them so); without it such a call fails with hipErrorInvalidValue.
 hipError_t launch_attention(const float* q, const float* k, const float* v, float* out, int T, int pos0,
                             const int* pos_dev, int n_heads, int n_kv, int hd, float* kc, float* vc, int max_ctx,
                             const float* rcos, const float* rsin, hipStream_t s, int8_t* xq = nullptr,

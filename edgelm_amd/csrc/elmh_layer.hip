@@ -1835,12 +1835,6 @@ hipError_t launch_rmsnorm(const float* x, const float* w, float* y, int rows, in
   return hipGetLastError();
 }
 
-size_t attention_global_score_bytes(int T, int pos0, bool pos_dev, int n_heads, int hd, int max_ctx) {
-  const int n_cap = pos_dev ? max_ctx : pos0 + T;
-  if (attention_lds_bytes(hd, n_cap) <= kMaxAttnLds) return 0;
-  return (size_t)T * n_heads * (size_t)((n_cap + 63) & ~63) * sizeof(float);
-}
-
 template <int R>
 static hipError_t launch_attention_rows(const float* q, float* out, const float* kc, const float* vc, int T, int pos0, int grp,
                                         int n_kv, int hd, int max_ctx, const float* rcos, const float* rsin, int8_t* xq,
@@ -1873,18 +1867,16 @@ bool raise_lds_limit() {
   return true;
 }
 
-static bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
-
 hipError_t launch_attention(const float* q, const float* k, const float* v, float* out, int T, int pos0,
                             const int* pos_dev, int n_heads, int n_kv, int hd, float* kc, float* vc, int max_ctx,
                             const float* rcos, const float* rsin, hipStream_t s, int8_t* xq, float* xd, int Tpad,
                             bool* quantized, float* gscores) {
   if (quantized) *quantized = false;
-  // with the position in device memory the score buffer covers the whole cache
-  const int n_cap = pos_dev ? max_ctx : pos0 + T;  // score slots
   const int grp = n_heads / n_kv;
   const bool quant = xq && xd && quantized;
-  const AttnKernel route = attention_route({T, n_cap, pos_dev != nullptr, n_heads, n_kv, hd, quant, aligned16(kc)});
+  const AttnCall call = attention_call(T, pos0, pos_dev != nullptr, n_heads, n_kv, hd, kc, max_ctx, quant);
+  const AttnKernel route = attention_route(call);
+  const int n_cap = call.n_cap;
   // one token, and chunks on the head-size-64 prefill kernel: the append runs inside the attention
   // kernel; other chunks append every key first
   const bool fuse = T == 1;

@@ -14,6 +14,9 @@ using namespace elmh;
 extern "C" int attn(int T, int n_cap, int pos_dev, int nh, int nkv, int hd, int quant, int aligned) {
   return (int)attention_route({T, n_cap, pos_dev != 0, nh, nkv, hd, quant != 0, aligned != 0});
 }
+extern "C" size_t score_bytes(int T, int n_cap, int pos_dev, int nh, int nkv, int hd, int quant, int aligned) {
+  return attention_global_score_bytes({T, n_cap, pos_dev != 0, nh, nkv, hd, quant != 0, aligned != 0});
+}
 """
 STEP, ROWS4, ROWS8, PREFILL64, PREFILL, DECODE64, WHOLE, GLOBAL = range(8)
 
@@ -24,7 +27,9 @@ def routes(tmp_path_factory):
     (d / "shim.cpp").write_text(SHIM)
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I",
                     os.path.join(ROOT, "edgelm_amd", "csrc"), str(d / "shim.cpp"), "-o", str(d / "routes.so")], check=True)
-    return C.CDLL(str(d / "routes.so"))
+    lib = C.CDLL(str(d / "routes.so"))
+    lib.score_bytes.restype = C.c_size_t
+    return lib
 
 
 def test_attention_key_cache_off_16_bytes(routes):
@@ -39,3 +44,19 @@ def test_attention_key_cache_off_16_bytes(routes):
     assert routes.attn(1, 2048, 1, 32, 8, 128, 0, 0) == WHOLE
     assert routes.attn(1, 2048, 1, 32, 8, 128, 0, 1) == STEP
     assert routes.attn(256, 512, 0, 32, 8, 128, 0, 1) == ROWS8
+
+
+def test_attention_score_rows_only_where_they_are_used(routes):
+    """A call that keeps its score rows in LDS asks for no global ones (a step over 20 to 24 thousand positions: the step
+    kernel holds them where attention_kernel would not), and one on the kernel that uses them always does."""
+    assert routes.attn(1, 22000, 1, 32, 8, 128, 0, 1) == STEP and routes.score_bytes(1, 22000, 1, 32, 8, 128, 0, 1) == 0
+    assert routes.attn(1, 30000, 1, 32, 8, 128, 0, 1) == GLOBAL
+    assert routes.score_bytes(1, 30000, 1, 32, 8, 128, 0, 1) == 32 * 30016 * 4
+    for T in (1, 2, 64, 700):
+        for nh, nkv in ((9, 3), (32, 8)):
+            for hd in (16, 64, 128):
+                for quant in (0, 1) if T > 1 and hd == 64 else (0,):
+                    for n in range(T, 50000, 997):
+                        need = routes.attn(T, n, 0, nh, nkv, hd, quant, 1) == GLOBAL
+                        got = routes.score_bytes(T, n, 0, nh, nkv, hd, quant, 1)
+                        assert got == (T * nh * ((n + 63) // 64 * 64) * 4 if need else 0)
