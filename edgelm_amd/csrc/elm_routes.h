@@ -81,12 +81,15 @@ inline AttnKernel attention_route(const AttnCall& c) {
   //
   // A chunk of at most one (token, head) per CU: a 1024-thread workgroup each (32 heads of size 128 over 1000 cached
   // positions: 35 / 38 us for 2 / 8 tokens, against 51 us with rows of four in 256-thread workgroups; 16 tokens 55 against
-  // 52). At head size 64 only where no GEMM operand is asked for (8 tokens of 9 heads over 300 positions: 13.7 against 17.9
-  // us with attention_prefill64_kernel). One token: always, but for the head-size-64 kernel's caches (it takes the step's
-  // rows before it knows the position: 6.0 against 8.6 us at 200 positions, 15.4 against 19.9 at 700).
+  // 52). At head size 64 only where no GEMM operand is asked for, and past 128 positions, where attention_prefill64_kernel, which
+  // has the append inside, starts a second chunk of rows: it takes 7.0 / 7.6 / 9.8 / 10.3 / 12.0 / 13.3 / 34.6 us for 8 tokens of 9
+  // heads over 96 / 128 / 144 / 192 / 256 / 288 / 1000 positions, the append and the step kernel 8.5 / 8.9 / 9.1 / 9.8 / 10.8 / 11.2
+  // / 21.9 (32 heads over 8 kv heads, 8 tokens: 7.1 / 7.7 / 9.7 / 10.4 / 12.2 / 13.4 / 35.6 and 8.2 / 8.6 / 9.0 / 9.5 / 10.4 / 11.2
+  // / 23.2; 2 to 64 tokens alike). One token: always, but for the head-size-64 kernel's caches (it takes the step's rows before it
+  // knows the position: 6.0 against 8.6 us at 200 positions, 15.4 against 19.9 at 700).
   const bool step_fits = c.aligned && grp < 65536 && attention_step_lds_bytes(c.hd, c.n_cap) <= kMaxAttnLds;
   const bool step = step_fits && (fuse ? c.hd != 64 || attention_decode_lds_bytes(c.n_cap) > kMaxAttnLds
-                                       : !c.pos_dev && pairs <= 256 && (c.hd != 64 || !c.quant));
+                                       : !c.pos_dev && pairs <= 256 && (c.hd != 64 || (!c.quant && c.n_cap > kPfRows)));
   if (step) return AttnKernel::kStep;
   // Longer chunks: attention_rows_kernel, at head size 64 from 4096 (token, head) pairs on (9 heads: 512 tokens 31 against
   // 48 us with attention_prefill64_kernel, 128 tokens 11 against 8.4; 32 heads, 64 tokens at 600 positions 34 against 32).

@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 # (n_heads, n_kv, head_dim, max_ctx, pos0, T): 4 rows (T * heads / 8 < 1024), 8 rows, one workgroup per row (<= 256)
 SHAPES = [(8, 2, 128, 400, 0, 65), (12, 4, 96, 330, 250, 33), (6, 2, 100, 90, 3, 61), (5, 1, 256, 100, 15, 60), (16, 4, 4, 70, 0, 64),
           (32, 8, 64, 300, 1, 257), (32, 8, 20, 300, 0, 257),
-          (8, 8, 80, 1100, 1020, 3), (4, 1, 128, 80, 0, 64), (9, 3, 64, 80, 60, 5)]
+          (8, 8, 80, 1100, 1020, 3), (4, 1, 128, 80, 0, 64),
+          (9, 3, 64, 80, 60, 5), (9, 3, 64, 200, 126, 2), (9, 3, 64, 200, 126, 3), (4, 1, 64, 400, 300, 64)]  # 128 positions, past them
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=["x".join(map(str, s)) for s in SHAPES])

@@ -60,3 +60,19 @@ def test_attention_score_rows_only_where_they_are_used(routes):
                         need = routes.attn(T, n, 0, nh, nkv, hd, quant, 1) == GLOBAL
                         got = routes.score_bytes(T, n, 0, nh, nkv, hd, quant, 1)
                         assert got == (T * nh * ((n + 63) // 64 * 64) * 4 if need else 0)
+
+
+@pytest.mark.parametrize("nh,nkv", [(9, 3), (14, 2), (32, 8), (4, 1)])
+def test_attention_short_prompts_append_inside(routes, nh, nkv):
+    """Head size 64, a chunk of few (token, head) pairs without a GEMM operand (a default Session's short prompt): one launch
+    with the append inside up to 128 positions, the append and the step kernel past them."""
+    for T in (2, 3, 5, 8, 17, 28, 64):
+        if T * nh > 256:
+            continue
+        for n in (T, 64, 96, 128):
+            assert n < T or routes.attn(T, n, 0, nh, nkv, 64, 0, 1) == PREFILL64
+        for n in (129, 144, 192, 300, 700):
+            assert routes.attn(T, n, 0, nh, nkv, 64, 0, 1) == STEP
+        for n in (64, 192, 300):  # with the GEMM's operand: the kernel that writes it
+            assert routes.attn(T, n, 0, nh, nkv, 64, 1, 1) == PREFILL64
+        assert routes.attn(T, 100, 0, nh, nkv, 128, 0, 1) == STEP  # other head sizes: always
