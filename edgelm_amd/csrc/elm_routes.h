@@ -113,4 +113,45 @@ inline size_t attention_global_score_bytes(const AttnCall& c) {
   return (size_t)c.T * c.n_heads * (size_t)((c.n_cap + 63) & ~63) * sizeof(float);
 }
 
+// ---------------------------------------------------------------- int8 GEMM
+
+constexpr int kLds16MaxBlocks = 48;  // gemm_lds16_kernel: rows of at most this many 32-blocks (K <= 1536)
+
+// Whether gemm_split16_kernel (K split over a workgroup's waves) takes a GEMM of nb 32-blocks per row and T tokens that makes
+// `wgs` of its workgroups (row tiles in eights, times groups of 16 tokens). swiglu: gate and up; token: one scale per token;
+// ring: the ring kernel would take the call (gemm_wave16_kernel otherwise).
+// Its time goes with its workgroups; gemm_wave16_kernel's hardly does until it fills the chip, so there is a count past which it
+// is the faster one, higher the more a workgroup of the split has to gain. A workgroup walks K in whole rounds of 16 blocks, so
+// workgroups are counted with nb rounded up to those. Times in us, the other kernel's first, then the split's (256 CUs):
+//   q4, scale per block   4096 x 14336 at 16 / 64 / 128 / 256 tokens (256 / 1024 / 2048 / 4096 workgroups): 104 / 94 / 123 / 145, 22
+//                         / 56 / 104 / 231; 8192 x 2048 at 64 / 65 tokens (2048 / 2560): 24 / 24, 23 / 26
+//   q8, scale per block   4096 x 4096 at 96 / 112 / 128 tokens (1536 / 1792 / 2048): the split takes 0.82 / 0.93 / 1.02 of the
+//                         other's time; 2048 x 2048 at 192 / 256 (1536 / 2048) 0.92 / 1.13
+//   q4, scale per token   1536 x 1568 at 192 / 224 tokens (1152 / 1344 of 49 blocks): 15.8 / 15.9, 15.1 / 17.0; 2048 x 2048 at 192 /
+//                         256 (1536 / 2048) 0.95 / 1.14; 4096 x 4096 at 112 (1792) 0.90; 4096 x 14336 at 128 (2048) 0.90
+//   q8, scale per token   (no rescale: sums of integers) 4096 x 4096 / 4096 x 14336 at 128 tokens (2048): 0.80 / 0.65
+//   SwiGLU q4             14336 x 4096 at 16 / 17 to 32 tokens (896 / 1792): 0.9 / 1.05 (scale per block), 0.95 / 1.2 (per token);
+//                         1536 x 1568 at 128 / 160 (768 / 960 of 49 blocks): 0.94 / 1.08, 0.96 / 1.12
+//   SwiGLU q8, per token  4096 x 4096 at 64 tokens (1024) 0.80, 1536 x 1568 at 192 (1152 of 49 blocks) 0.82, 14336 x 4096 at 17 (1792)
+//                         0.99
+//   SwiGLU q8, per block  (82 KB of LDS: one workgroup per CU) 14336 x 4096 at 16 (896): 31.7, 45.3; 11008 x 4096 at 16 (688): 30.3,
+//                         35.1; 8192 x 4096 at 16 (512) 0.85; 2048 x 2048 at 64 / 65 (512 / 640) 0.96 / 1.26; 1536 x 1568 at 48 (288 of
+//                         49 blocks): 15.1, 15.8
+// More tokens over few rows fill the chip with the other's workgroups earlier (256 x 2048 q8 at 1536 tokens, 1536 workgroups 1.08; as
+// SwiGLU q4 at 1024 tokens, 1024 workgroups 1.05). The ring kernel, which serves what makes 128 tiles of 128 rows x 64 tokens, is
+// slower at few tokens: 16384 x 4096 at 16 tokens (1024 workgroups) 0.52 q4, 0.65 q8, SwiGLU 0.26 and 0.48; 32000 x 4096 at 16
+// (2000) 0.84 and 1.06, per token 0.76 and 1.00.
+inline bool gemm_split16_route(bool q8, bool swiglu, bool token, bool ring, int nb, int T, int64_t wgs) {
+  if (nb <= kLds16MaxBlocks) return false;
+  const int64_t load = wgs * ((nb + 15) / 16 * 16) / nb;
+  const bool many = T > (q8 && token ? 1024 : 768);
+  if (swiglu) {
+    if (q8 && !token && !ring) return load <= (many || nb < 64 ? 340 : 530);
+    return load <= (many ? 900 : q8 && token ? 1536 : 1200);
+  }
+  if (many) return load <= 1200;
+  if (q8) return load <= (!token ? 1840 : ring ? 1900 : 2100);
+  return load <= (!token || ring || nb >= 256 ? 2100 : nb >= 96 ? 1840 : 1700);
+}
+
 }  // namespace elmh

@@ -2034,7 +2034,6 @@ __global__ __launch_bounds__((64 * SplitLds<WDT, SW, TOK, G, D>::WAVES)) void ge
 // half of every block into the next GEMM's fragments with edgelm's rounding (act_quant_frag_kernel's
 // arithmetic: s = amax / 127, each value's rounding that of its division).
 __host__ __device__ constexpr int lds16_region_bytes(int bytes) { return (bytes + 1023) / 1024 * 1024; }
-constexpr int kLds16MaxBlocks = 48;  // K <= 1536
 constexpr int kLds16Ahead = 3;       // blocks read ahead; every region has room for them past nb
 template <int WDT, bool SW, bool TOK, bool QF = false>
 __host__ __device__ inline int gemm_lds16_bytes(int nb) {
@@ -3246,7 +3245,7 @@ static bool gemm_split16_launch(const GemmArgs& a, hipStream_t s) {
   };
   // one workgroup per CU: longer rounds (q4 4096 x 14336, 16 tokens 22.1 against 23.9 us), or for the per-token sums one more
   // slot (18.6 against 23.7 us); more: two slots of 16 blocks, so that two workgroups fit a CU (64 tokens 57 us; 70 with the
-  // longer rounds, 59 with three slots)
+  // longer rounds, 59 with three slots), except per-block q8 SwiGLU, whose 82 KB fit once
   using std::integral_constant;
   if (wgs <= 256) {
     if constexpr (TOK && WDT == WQ8) return go(integral_constant<int, 2>{}, integral_constant<int, 3>{});
@@ -3341,15 +3340,12 @@ static hipError_t gemm_go(const GemmArgs& a, int tiles, hipStream_t s) {
     wave32 = std::strcmp(ev, "wave32") == 0;
     lds16 = ev[0] == 'l';
   }
-  // A few tokens over long rows: K split over a workgroup's waves (gemm_split16_kernel) up to 2048 workgroups, 1200 with
-  // SwiGLU (each the work of two). Per-block q4, against the kernels below: 4096 x 14336 at 16 / 64 / 128 / 256 tokens (256 /
-  // 1024 / 2048 / 4096 workgroups) 22 / 57 / 103 / 214 us against 104 / 95 / 123 / 136; 4096 x 4096 10 / 21 / 35 / 69 against
-  // 32 / 32 / 38 / 44; 14336 x 4096 at 16 / 32 / 64 tokens 21 / 34 / 62 against 33 / 39 / 64. ELMH_GEMM_KERNEL=split forces
-  // it. Not for the fused multiply-adds of ELMH_FAST.
-  const int64_t split_wgs = gemm_split16_wgs<SW>(a);
+  // A few tokens over long rows: K split over a workgroup's waves (gemm_split16_route). ELMH_GEMM_KERNEL=split forces it. Not for
+  // the fused multiply-adds of ELMH_FAST.
   const char* const forced = getenv("ELMH_GEMM_KERNEL");
   const bool split = forced ? std::strcmp(forced, "split") == 0
-                            : a.nb > kLds16MaxBlocks && split_wgs <= (SW ? 1200 : 2048) && !getenv("ELMH_GEMM_TOKEN_TILE");
+                            : !getenv("ELMH_GEMM_TOKEN_TILE") &&
+                                  gemm_split16_route(WDT == WQ8, SW, TOK, !wave, a.nb, a.T, gemm_split16_wgs<SW>(a));
   if (split && !a.fast && a.H >= 4 && !(a.H & (a.H - 1)) && gemm_split16_launch<WDT, SW, TOK>(a, s)) return hipGetLastError();
   if (wave) {
     if (wave32)

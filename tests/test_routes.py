@@ -17,6 +17,9 @@ extern "C" int attn(int T, int n_cap, int pos_dev, int nh, int nkv, int hd, int 
 extern "C" size_t score_bytes(int T, int n_cap, int pos_dev, int nh, int nkv, int hd, int quant, int aligned) {
   return attention_global_score_bytes({T, n_cap, pos_dev != 0, nh, nkv, hd, quant != 0, aligned != 0});
 }
+extern "C" int split16(int q8, int sw, int tok, int ring, int nb, int T, long wgs) {
+  return gemm_split16_route(q8 != 0, sw != 0, tok != 0, ring != 0, nb, T, wgs);
+}
 """
 STEP, ROWS4, ROWS8, PREFILL64, PREFILL, DECODE64, WHOLE, GLOBAL = range(8)
 
@@ -76,3 +79,31 @@ def test_attention_short_prompts_append_inside(routes, nh, nkv):
         for n in (64, 192, 300):  # with the GEMM's operand: the kernel that writes it
             assert routes.attn(T, n, 0, nh, nkv, 64, 1, 1) == PREFILL64
         assert routes.attn(T, 100, 0, nh, nkv, 128, 0, 1) == STEP  # other head sizes: always
+
+
+# (rows, K, tokens, faster with K split over the waves?) by (q8, SwiGLU, per-token scale), the measured calls nearest to where
+# the two kernels cross; the rows of a 16 x 16 tile grid counted in eights
+SPLIT = {
+    (0, 0, 0): [(4096, 14336, 16, 1), (4096, 14336, 128, 1), (4096, 14336, 256, 0), (8192, 2048, 64, 1), (8192, 2048, 65, 0),
+                (1536, 1568, 320, 0), (64, 2048, 4096, 0), (32000, 4096, 16, 1)],
+    (1, 0, 0): [(4096, 4096, 112, 1), (4096, 4096, 128, 0), (2048, 2048, 192, 1), (2048, 2048, 256, 0), (32000, 4096, 8, 0),
+                (16384, 4096, 16, 1), (128, 1568, 2048, 0), (1024, 14336, 512, 0)],
+    (0, 0, 1): [(1536, 1568, 192, 1), (1536, 1568, 224, 0), (8192, 2048, 64, 0), (1024, 4096, 512, 0), (4096, 14336, 128, 1),
+                (32000, 4096, 16, 1)],
+    (1, 0, 1): [(4096, 14336, 128, 1), (16384, 4096, 32, 0), (256, 2048, 1536, 0), (4096, 4096, 256, 0)],
+    (0, 1, 0): [(14336, 4096, 16, 1), (14336, 4096, 17, 0), (576, 1568, 384, 0), (1536, 1568, 128, 1), (256, 2048, 1024, 0),
+                (16384, 4096, 16, 1)],
+    (1, 1, 0): [(14336, 4096, 16, 0), (14336, 4096, 5, 0), (11008, 4096, 16, 0), (6144, 4096, 16, 1), (2048, 2048, 64, 1),
+                (2048, 2048, 65, 0), (4096, 4096, 32, 1), (4096, 4096, 33, 0), (1536, 1568, 48, 0), (16384, 4096, 16, 1)],
+    (0, 1, 1): [(14336, 4096, 16, 1), (576, 1568, 384, 0), (1536, 1568, 160, 0), (256, 2048, 1024, 0), (4096, 4096, 64, 1)],
+    (1, 1, 1): [(14336, 4096, 16, 1), (4096, 4096, 64, 1), (128, 1568, 1536, 0), (1536, 1568, 320, 0)],
+}
+
+
+@pytest.mark.parametrize("kind", SPLIT, ids=lambda k: f"q{8 if k[0] else 4}{'-swiglu' * k[1]}{'-token' * k[2]}")
+def test_gemm_split_over_waves_where_it_is_faster(routes, kind):
+    for n, k, T, split in SPLIT[kind]:
+        wgs = -(-(-(-n // 16)) // 8) * 8 * -(-T // 16)
+        ring = -(-n // 128) * -(-T // 64) >= 128
+        assert bool(routes.split16(*kind, ring, k // 32, T, C.c_long(wgs))) == bool(split), (n, k, T)
+    assert not routes.split16(*kind, 0, 48, 16, C.c_long(8))  # short rows: gemm_lds16_kernel
