@@ -154,4 +154,57 @@ inline bool gemm_split16_route(bool q8, bool swiglu, bool token, bool ring, int 
   return load <= (!token || ring || nb >= 256 ? 2100 : nb >= 96 ? 1840 : 1700);
 }
 
+// ---------------------------------------------------------------- f32-activation GEMM (more than one token)
+
+// Rows x tokens of a workgroup: gemm_f32act_kernel, and the tiles of gemm_f32act_tile_kernel
+enum class F32Gemm { k64x2, k16x8, k32x16, k64x16, k64x32 };
+
+// N: the output rows of the n targets (SwiGLU: the gate's). Times in us at K = 4096 q4 unless said otherwise.
+//
+// Tiles: the largest that makes at least two workgroups per CU (one for 32 x 16), else 16 x 8: at 4096 rows and 256 / 128 / 64 / 32
+// / 16 tokens 64 x 32 tiles take 189 / 114 / 109 / 105 / 95, 64 x 16 220 / 115 / 71 / 68 / 67, 32 x 16 240 / 124 / 65 / 41 / 40,
+// 16 x 8 343 / 179 / 95 / 50 / 29. A token tile that is mostly empty has waves that only stage: 64 x 32 needs more than 16 tokens
+// (49152 x 576 at 2 / 8 / 16 tokens 35 / 36 / 38, with 64 x 16 26 / 26 / 32) and, with q8 weights, up to 64 tokens, more than half of
+// its last tile (32768 x 1024 at 33 / 48: 124 / 129, 64 x 16 91 / 95; q4 96 / 101 and 88 / 92); up to 5 tokens, and 6 below K = 2048, there are 16 x 8 and
+// 64 x 16 only (8192 x 2048 at 2 to 5: 15.4, 32 x 16 19.5; 24576 x 576 at 5: 13.6 and 15.8; 14336 x 4096 at 6: 44 and 42). SwiGLU holds both selections, so at most
+// 32 x 16 (3648 x 1088, 175 tokens, with its down projection: 148, 185 with 64 x 16), and 16 x 8 up to 384 of those: between 256
+// and 384 they run in two rounds of the CUs (1536 x 576 q8, 93 tokens, 288 of them, with its down projection: 35 against 42; 4096 rows
+// at 17 tokens, 256 half-empty ones: 56 against 60; with whole tiles in one round they would be the faster, 4096 rows at 32 tokens 86
+// against 73, 2048 x 2048 at 64 46 against 39).
+//
+// gemm_f32act_kernel (every weight dequantized for each pair of tokens, but all lanes at work): few tokens over many rows, and the
+// shortest rows at a middling number of outputs, where the tiles' staging is not repaid. Its time first, then the tiles':
+//   2 tokens   16384 x 576 / 1024 10.0 / 15.7 and 10.8 / 13.6; 24576 x 576 / 1024 / 2048 10.0 / 16.3 / 38.6 and 13.3 / 18.4 / 35;
+//              32000 x 4096 72 and 82 (SwiGLU 93 and 124); 49152 x 576 12.5 and 26; 128256 x 2048 82 and 152; 14336 x 4096 65 and 40
+//   3 or 4     24576 x 256 / 576 / 1024 6.6 / 10.8 / 21.2 and 8.8 / 13.3 / 20.5; 49152 x 576 18.9 and 25.5 (SwiGLU 34.7 and 37.1);
+//              32000 x 4096 89 and 81; 128256 x 2048 142 and 150 to 160
+//   5, 6       24576 x 256 8.2 and 8.8, x 576 15.8 and 13.6
+//   8          49152 x 64 / 160 / 192 8.4 / 12.0 / 14.5 and 11.2 / 14.7 / 15.2
+//   17         16384 x 192 11.2 and 12.2, 49152 x 192 as SwiGLU 56 and 62 (a second tile of one token)
+//   K = 64     4096 x 33 tokens 5.1 and 6.0, 1536 x 93 5.0 and 5.8; 512 x 64 3.9 and 3.4, 4096 x 128 10.1 and 9.0
+inline F32Gemm f32_gemm_route(bool q8, bool swiglu, int T, int K, const int* N, int n) {
+  auto groups = [&](int rows) {
+    int64_t g = 0;
+    for (int i = 0; i < n; ++i) g += (N[i] + rows - 1) / rows;
+    return g;
+  };
+  const int64_t rows = groups(1), outputs = rows * T;
+  const bool many = rows > 24576;
+  bool pair = false;
+  if (rows <= 12288) pair = K <= 64 && outputs >= 40000 && outputs <= (swiglu ? 240000 : 400000);
+  else if (T <= 2) pair = K <= 640 || many || (K < 2048 && rows > 20480);
+  else if (T <= 4) pair = K <= (many || !swiglu ? 640 : 384) || rows > 98304;
+  else if (T <= 6) pair = K <= (swiglu ? 128 : 256);
+  else if (T <= 8) pair = K <= (swiglu ? 96 : 192);
+  else if (T <= 12) pair = K <= 64 && !swiglu;
+  else if (T > 16 && T <= 20) pair = swiglu ? K <= (many ? 320 : 192) : !many && K <= 192;
+  else if (T <= 24) pair = K <= 64 && !many && !swiglu;
+  if (pair && groups(64) <= 65535) return F32Gemm::k64x2;
+  auto wgs = [&](int r, int t) { return groups(r) * ((T + t - 1) / t); };
+  if (T <= (K < 2048 ? 6 : 5)) return !swiglu && wgs(64, 16) >= 512 ? F32Gemm::k64x16 : F32Gemm::k16x8;
+  if (!swiglu && T > 16 && (!q8 || T > 64 || (T - 1) % 32 >= 16) && wgs(64, 32) >= 512) return F32Gemm::k64x32;
+  if (!swiglu && wgs(64, 16) >= 512) return F32Gemm::k64x16;
+  return wgs(32, 16) >= (swiglu ? 384 : 256) ? F32Gemm::k32x16 : F32Gemm::k16x8;
+}
+
 }  // namespace elmh

@@ -2788,7 +2788,144 @@ __device__ __forceinline__ float deq1(const uint8_t* __restrict__ data, const fl
   return (float)((int)(e >= 16 ? byte >> 4 : byte & 0x0F) - 8) * scales[item];
 }
 
-// The chains are independent, so they run from a tile in LDS: a workgroup is 16 RY rows x 8 TX tokens. Lane 4 m + c of a wave runs chain c of
+// The chains are independent. A few tokens over many rows, and the shortest rows (f32_gemm_route): four lanes take one (row,
+// kF32TT tokens) tile, a chain each; a workgroup is 64 rows x kF32TT tokens, so that every lane has work down to 2 tokens. x is
+// staged through LDS by chain ([token][chain][k / 4], so a lane reads four of its chain's values at once), and the row's four
+// lanes read the same 16 weight bytes, each using its own four.
+constexpr int kF32TT = 2;
+constexpr int kF32Chunk = 2048;
+constexpr int kF32ChainStride = kF32Chunk / 4 + 4;  // floats; the +4 spreads the staging writes over banks
+
+// The 16 weight bytes that hold elements i .. i + 15 of row n (i % 16 == 0) and their scale
+struct WChunk {
+  uint4 q;
+  float s;
+};
+template <int WDT>
+__device__ __forceinline__ WChunk load_chunk(const uint8_t* __restrict__ data, const float* __restrict__ scales,
+                                             int64_t nbase, int H, int i, int n) {
+  const int64_t item = nbase + (int64_t)(i >> 5) * H;
+  if (WDT == WQ8) return {*reinterpret_cast<const uint4*>(data + item * 32 + (i & 31)), scales[n]};
+  return {*reinterpret_cast<const uint4*>(data + item * 16), scales[item]};  // the group: byte m holds m, m + 16
+}
+// chain c's four dequantized weights of the chunk: elements i + c + 4m, m = 0 .. 3
+template <int WDT>
+__device__ __forceinline__ float4 chunk_chain(const WChunk& w, int i, int c) {
+  float4 r;
+  if (WDT == WQ8) {
+    r.x = (float)(int8_t)((w.q.x >> (8 * c)) & 0xFF) * w.s;
+    r.y = (float)(int8_t)((w.q.y >> (8 * c)) & 0xFF) * w.s;
+    r.z = (float)(int8_t)((w.q.z >> (8 * c)) & 0xFF) * w.s;
+    r.w = (float)(int8_t)((w.q.w >> (8 * c)) & 0xFF) * w.s;
+  } else {
+    const int sh = 8 * c + ((i & 31) >= 16 ? 4 : 0);
+    r.x = (float)((int)((w.q.x >> sh) & 0x0F) - 8) * w.s;
+    r.y = (float)((int)((w.q.y >> sh) & 0x0F) - 8) * w.s;
+    r.z = (float)((int)((w.q.z >> sh) & 0x0F) - 8) * w.s;
+    r.w = (float)((int)((w.q.w >> sh) & 0x0F) - 8) * w.s;
+  }
+  return r;
+}
+constexpr int kF32Ahead = 4;  // 16-element steps whose weights are in flight
+
+template <int WDT, bool SW>
+__global__ __launch_bounds__(256) void gemm_f32act_kernel(const F32Args a) {
+  __shared__ __align__(16) float sxp[kF32TT][4][kF32ChainStride];
+  int grp = blockIdx.y;
+  const GemvTarget tg = f32_target<SW>(a, grp);
+  const int K = a.K, K4 = K & ~3, H = a.H, nb = a.nb, T = a.T;
+  const int t0 = blockIdx.x * kF32TT, c = threadIdx.x & 3;
+  const int n = grp * 64 + (threadIdx.x >> 2);  // rows past N: padding (rows_pad % 64 == 0)
+  const int64_t nbase = (int64_t)(n / H) * nb * H + (n % H);
+  float s[kF32TT], su[kF32TT];
+#pragma unroll
+  for (int t = 0; t < kF32TT; ++t) s[t] = su[t] = 0.f;
+  for (int k0 = 0; k0 < K4; k0 += kF32Chunk) {
+    const int klen = min(kF32Chunk, K4 - k0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kF32TT * kF32Chunk; i += 256) {
+      const int t = i / kF32Chunk, k = i - t * kF32Chunk;
+      if (k < klen) sxp[t][k & 3][k >> 2] = t0 + t < T ? a.x[(int64_t)(t0 + t) * K + k0 + k] : 0.f;
+    }
+    __syncthreads();
+    // the chunk's 16-element steps; each step's weights are loaded kF32Ahead steps before it
+    const int nst = klen >> 4;
+    WChunk wr[kF32Ahead], ur[kF32Ahead];
+#pragma unroll
+    for (int u = 0; u < kF32Ahead; ++u)
+      if (u < nst) {
+        wr[u] = load_chunk<WDT>(tg.data, tg.scales, nbase, H, k0 + 16 * u, n);
+        if (SW) ur[u] = load_chunk<WDT>(a.tg[1].data, a.tg[1].scales, nbase, H, k0 + 16 * u, n);
+      }
+    for (int s0 = 0; s0 < nst; s0 += kF32Ahead) {
+#pragma unroll
+      for (int u = 0; u < kF32Ahead; ++u) {
+        const int st = s0 + u, ii = k0 + 16 * st;
+        if (st < nst) {
+          const float4 w = chunk_chain<WDT>(wr[u], ii, c);
+          const float4 wu = SW ? chunk_chain<WDT>(ur[u], ii, c) : w;
+          if (st + kF32Ahead < nst) {
+            wr[u] = load_chunk<WDT>(tg.data, tg.scales, nbase, H, ii + 16 * kF32Ahead, n);
+            if (SW) ur[u] = load_chunk<WDT>(a.tg[1].data, a.tg[1].scales, nbase, H, ii + 16 * kF32Ahead, n);
+          }
+#pragma unroll
+          for (int t = 0; t < kF32TT; ++t) {
+            const float4 xv = *reinterpret_cast<const float4*>(&sxp[t][c][(ii - k0) >> 2]);
+            s[t] = s[t] + xv.x * w.x;
+            s[t] = s[t] + xv.y * w.y;
+            s[t] = s[t] + xv.z * w.z;
+            s[t] = s[t] + xv.w * w.w;
+            if (SW) {
+              su[t] = su[t] + xv.x * wu.x;
+              su[t] = su[t] + xv.y * wu.y;
+              su[t] = su[t] + xv.z * wu.z;
+              su[t] = su[t] + xv.w * wu.w;
+            }
+          }
+        }
+      }
+    }
+    int i = k0 + 16 * nst;
+    for (; i < k0 + klen; i += 4) {  // the last chunk's steps past its last 16-element run
+      const float w = deq1<WDT>(tg.data, tg.scales, nbase, H, i + c, n);
+      const float wu = SW ? deq1<WDT>(a.tg[1].data, a.tg[1].scales, nbase, H, i + c, n) : w;
+#pragma unroll
+      for (int t = 0; t < kF32TT; ++t) {
+        const float xv = sxp[t][c][(i - k0) >> 2];
+        s[t] = s[t] + xv * w;
+        if (SW) su[t] = su[t] + xv * wu;
+      }
+    }
+  }
+  if (c == 0)
+    for (int i = K4; i < K; ++i) {  // tail (K % 4) into the first chain
+      const float w = deq1<WDT>(tg.data, tg.scales, nbase, H, i, n);
+      const float wu = SW ? deq1<WDT>(a.tg[1].data, a.tg[1].scales, nbase, H, i, n) : w;
+#pragma unroll
+      for (int t = 0; t < kF32TT; ++t) {
+        const float xv = t0 + t < T ? a.x[(int64_t)(t0 + t) * K + i] : 0.f;
+        s[t] = s[t] + xv * w;
+        if (SW) su[t] = su[t] + xv * wu;
+      }
+    }
+#pragma unroll
+  for (int t = 0; t < kF32TT; ++t) {
+    const float p = s[t] + __shfl_xor(s[t], 1);  // lane 0: s0 + s1, lane 2: s2 + s3
+    const float dot = p + __shfl_xor(p, 2);
+    float out;
+    if (SW) {
+      const float pu = su[t] + __shfl_xor(su[t], 1);
+      const float g = 0.f + dot;
+      const float u = 0.f + (pu + __shfl_xor(pu, 2));
+      out = silu_exact(g) * u;
+    } else {
+      out = (t0 + t < T && tg.res ? tg.res[(int64_t)(t0 + t) * tg.N + n] : 0.f) + dot;
+    }
+    if (c == 0 && n < tg.N && t0 + t < T) tg.y[(int64_t)(t0 + t) * tg.N + n] = out;
+  }
+}
+
+// The others run from a tile in LDS: a workgroup is 16 RY rows x 8 TX tokens. Lane 4 m + c of a wave runs chain c of
 // rows m, m + 16, .. for the wave's TX tokens (gate and up with SW), so that a quad's four lanes hold one (row, token)'s
 // four chains. 16 P k's per step are staged in two buffers with one barrier per step: the weights dequantized once for the
 // workgroup, both operands as 16-byte slots of one chain's next four values (k = 16 h + 4 u + c, u = 0 .. 3), [h][item][c],
@@ -3481,17 +3618,29 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
       gemv_f32act_q8_kernel<false><<<groups, 64, lds, s>>>(b);
     }
   } else {
-    // The largest tile that makes at least two workgroups per CU (one for 32 rows x 16 tokens), else 16 rows x 8 tokens: at
-    // 4096 x 4096 q4 and 256 / 128 / 64 / 32 / 16 tokens 64 x 32 tiles take 189 / 114 / 109 / 105 / 95 us, 64 x 16 220 / 115 /
-    // 71 / 68 / 67, 32 x 16 240 / 124 / 65 / 41 / 40, 16 x 8 343 / 179 / 95 / 50 / 29. SwiGLU holds both selections, so at most
-    // 32 x 16 (3648 x 1088, 175 tokens, with its down projection: 148 us, 185 with 64 x 16), and 16 x 8 up to 384 of those (1536 x
-    // 576 q8, 93 tokens, with its down projection: 35 against 42 us).
-    auto wgs = [&](int ry, int tx) {
-      int64_t g = 0;
-      for (int i = 0; i < n; ++i) g += (a.tg[i].N + 16 * ry - 1) / (16 * ry);
-      return g * ((a.T + kF32TWaves * tx - 1) / (kF32TWaves * tx));
-    };
-    const int64_t big = 512, mid = swiglu ? 384 : 256;
+    int tn[kMaxTargets];
+    for (int i = 0; i < n; ++i) tn[i] = a.tg[i].N;
+    const F32Gemm route = f32_gemm_route(dtype == WQ8, swiglu != 0, a.T, a.K, tn, n);
+    if (route == F32Gemm::k64x2) {
+      // grid x: kF32TT-token tiles (consecutive workgroups share their weight rows), y: 64-row groups
+      F32Args b = a;
+      int groups = 0;
+      for (int i = 0; i < n; ++i) {
+        b.tile_start[i] = groups;
+        groups += (a.tg[i].N + 63) / 64;
+      }
+      b.tile_start[n] = groups;
+      if (groups < 1 || groups > 65535) return hipErrorInvalidValue;
+      const dim3 grid((a.T + kF32TT - 1) / kF32TT, groups);
+      if (dtype == WQ8) {
+        if (swiglu) gemm_f32act_kernel<WQ8, true><<<grid, 256, 0, s>>>(b);
+        else gemm_f32act_kernel<WQ8, false><<<grid, 256, 0, s>>>(b);
+      } else {
+        if (swiglu) gemm_f32act_kernel<WQ4, true><<<grid, 256, 0, s>>>(b);
+        else gemm_f32act_kernel<WQ4, false><<<grid, 256, 0, s>>>(b);
+      }
+      return hipGetLastError();
+    }
     auto go = [&](auto ry, auto tx, auto pp) {
       constexpr int RY = decltype(ry)::value, TX = decltype(tx)::value, P = decltype(pp)::value;
       F32Args b = a;
@@ -3516,12 +3665,12 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
       return hipGetLastError();
     };
     using std::integral_constant;
-    if (!swiglu && wgs(4, 4) >= big)
-      return go(integral_constant<int, 4>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{});
-    if (!swiglu && wgs(4, 2) >= big)
-      return go(integral_constant<int, 4>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
-    if (wgs(2, 2) >= mid) return go(integral_constant<int, 2>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
-    return go(integral_constant<int, 1>{}, integral_constant<int, 1>{}, integral_constant<int, 8>{});
+    switch (route) {
+      case F32Gemm::k64x32: return go(integral_constant<int, 4>{}, integral_constant<int, 4>{}, integral_constant<int, 4>{});
+      case F32Gemm::k64x16: return go(integral_constant<int, 4>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+      case F32Gemm::k32x16: return go(integral_constant<int, 2>{}, integral_constant<int, 2>{}, integral_constant<int, 8>{});
+      default: return go(integral_constant<int, 1>{}, integral_constant<int, 1>{}, integral_constant<int, 8>{});
+    }
   }
   return hipGetLastError();
 }

@@ -19,8 +19,8 @@ def weight(r, n, k, dt):
     return O.make_weight(r.normal(0, 0.05, (n, k)).astype(np.float32), dt)
 
 
-# (rows, K, T): 64 x 32 tiles (512 workgroups), 64 x 16, 32 x 16, 16 x 8
-TILES = [(2000, 96, 505), (1030, 160, 490), (1000, 288, 126), (70, 544, 9), (33, 2080, 2), (17, 32, 3)]
+# (rows, K, T): 64 x 32 tiles (512 workgroups; two steps and six, which use both buffers again), 64 x 16, 32 x 16, 16 x 8
+TILES = [(2000, 96, 505), (2000, 352, 505), (1030, 160, 490), (1000, 288, 126), (70, 544, 9), (33, 2080, 2), (17, 32, 3)]
 
 
 @pytest.mark.parametrize("shape", TILES, ids=["x".join(map(str, s)) for s in TILES])
@@ -42,6 +42,30 @@ def test_f32act_gemm_tiles(ctx, dt, shape):
         assert bits_equal(ctx.swiglu(x, dws[0], du, act=E.ACT_F32), O.cpu_swiglu(x, ws[0], wu, act_quant=False)), f"swiglu K={kk}"
         for d in dws + [du]:
             d.free()
+
+
+# (rows, K, T): pairs of tokens (gemm_f32act_kernel), K past its 2048-element chunk, K % 4 and an odd last token, several row groups
+PAIRS = [(12300, 90, 3), (24600, 2077, 2), (1540, 61, 33), (16400, 37, 7)]
+
+
+@pytest.mark.parametrize("shape", PAIRS, ids=["x".join(map(str, s)) for s in PAIRS])
+@pytest.mark.parametrize("dt", [O.Q8, O.Q4])
+def test_f32act_gemm_pairs_of_tokens(ctx, dt, shape):
+    n, k, T = shape
+    k = k if dt == O.Q8 else k // 32 * 32
+    r = np.random.default_rng(n + k)
+    ws = [weight(r, n, k, dt), weight(r, 40, k, dt)]
+    x = r.normal(0, 1, (T, k)).astype(np.float32)
+    res = r.normal(0, 1, (T, n)).astype(np.float32)
+    dws = [up(ctx, w) for w in ws]
+    print(f"[gpu] f32act gemm pairs of tokens dt={dt} {n}x{k} T={T}", flush=True)
+    for g, w in zip(ctx.matmul(x, dws, [res, None], act=E.ACT_F32), O.cpu_matmul(x, ws, [res, None], act_quant=False)):
+        assert bits_equal(g, w)
+    wu = weight(r, n, k, dt)
+    du = up(ctx, wu)
+    assert bits_equal(ctx.swiglu(x, dws[0], du, act=E.ACT_F32), O.cpu_swiglu(x, ws[0], wu, act_quant=False))
+    for d in dws + [du]:
+        d.free()
 
 
 def test_f32act_gemm_rows_shorter_than_a_chain(ctx):

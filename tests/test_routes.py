@@ -20,6 +20,7 @@ extern "C" size_t score_bytes(int T, int n_cap, int pos_dev, int nh, int nkv, in
 extern "C" int split16(int q8, int sw, int tok, int ring, int nb, int T, long wgs) {
   return gemm_split16_route(q8 != 0, sw != 0, tok != 0, ring != 0, nb, T, wgs);
 }
+extern "C" int f32gemm(int q8, int sw, int T, int K, const int* N, int n) { return (int)f32_gemm_route(q8 != 0, sw != 0, T, K, N, n); }
 """
 STEP, ROWS4, ROWS8, PREFILL64, PREFILL, DECODE64, WHOLE, GLOBAL = range(8)
 
@@ -107,3 +108,40 @@ def test_gemm_split_over_waves_where_it_is_faster(routes, kind):
         ring = -(-n // 128) * -(-T // 64) >= 128
         assert bool(routes.split16(*kind, ring, k // 32, T, C.c_long(wgs))) == bool(split), (n, k, T)
     assert not routes.split16(*kind, 0, 48, 16, C.c_long(8))  # short rows: gemm_lds16_kernel
+
+
+R64X2, R16X8, R32X16, R64X16, R64X32 = range(5)
+
+
+def f32gemm(routes, rows, K, T, q8=0, sw=0):
+    rows = [rows] if isinstance(rows, int) else rows
+    return routes.f32gemm(q8, sw, T, K, (C.c_int * len(rows))(*rows), len(rows))
+
+
+@pytest.mark.parametrize("q8", [0, 1])
+@pytest.mark.parametrize("sw", [0, 1])
+def test_f32_gemm_few_tokens(routes, q8, sw):
+    """Two to a few tokens: pairs of tokens where the rows are many, and no tile whose waves mostly stage only."""
+    for n, k, T, pairs in [(49152, 576, 2, 1), (49152, 576, 4, 1), (49152, 576, 5, 0), (49152, 576, 8, 0), (128256, 2048, 2, 1),
+                           (128256, 2048, 4, 1), (128256, 2048, 5, 0), (32000, 4096, 2, 1), (32000, 4096, 3, 0), (32768, 1024, 2, 1), (24576, 576, 2, 1),
+                           (16384, 1024, 2, 0), (14336, 4096, 2, 0), (12288, 576, 2, 0), (4096, 4096, 2, 0), (1536, 576, 2, 0),
+                           (16384, 256, 4, 1), (576, 576, 4, 0)]:
+        r = f32gemm(routes, n, k, T, q8, sw)
+        assert (r == R64X2) == bool(pairs), (n, k, T)
+        assert r != R64X32
+        assert T > 5 or r in (R64X2, R16X8, R64X16), (n, k, T)
+    assert f32gemm(routes, [4096, 1024, 1024], 4096, 2, q8, sw) == R16X8
+    assert f32gemm(routes, 18432, 576, 6, q8, sw) == R16X8 and f32gemm(routes, 14336, 4096, 6, q8, sw) == R32X16
+
+
+def test_f32_gemm_tiles(routes):
+    for T, tile in [(256, R64X32), (128, R64X16), (64, R32X16), (32, R32X16), (16, R16X8), (2, R16X8)]:
+        assert f32gemm(routes, 4096, 4096, T) == tile, T
+    for T, tile in [(16, R64X16), (17, R64X32), (32, R64X32), (33, R64X32), (65, R64X32)]:
+        assert f32gemm(routes, 49152, 576, T) == tile, T
+    for T, tile in [(17, R64X32), (32, R64X32), (33, R64X16), (48, R64X16), (49, R64X32), (65, R64X32)]:  # q8: the last tile's fill
+        assert f32gemm(routes, 49152, 576, T, q8=1) == tile, T
+    assert f32gemm(routes, 1536, 576, 93, q8=1, sw=1) == R16X8 and f32gemm(routes, 4096, 4096, 64, sw=1) == R32X16
+    for k, T, n, pairs in [(64, 33, 4096, 1), (64, 93, 1536, 1), (64, 64, 512, 0), (64, 256, 4096, 0), (96, 33, 4096, 0)]:
+        assert (f32gemm(routes, n, k, T) == R64X2) == bool(pairs), (n, k, T)
+    assert f32gemm(routes, 65536 * 64, 32, 2) != R64X2  # more row groups than a grid's second dimension takes
