@@ -207,4 +207,40 @@ inline F32Gemm f32_gemm_route(bool q8, bool swiglu, int T, int K, const int* N, 
   return wgs(32, 16) >= (swiglu ? 384 : 256) ? F32Gemm::k32x16 : F32Gemm::k16x8;
 }
 
+// ---------------------------------------------------------------- f32-activation q4 GEMV (one token)
+
+// gemv_f32act_q4_wide_kernel: nb groups per row spread over a workgroup's threads (256 up to 256 groups, which then hold several
+// sets of rows; else nb rounded up to whole waves), 8 rows each
+constexpr int kF32QRows = 8;
+inline bool f32q4_wide_ok(int nb, int H) { return nb > 64 && nb <= 512 && H >= kF32QRows && H % kF32QRows == 0; }
+inline int f32q4_wide_sets(int nb) { return nb <= 256 ? 256 / nb : 1; }
+inline int f32q4_wide_threads(int nb) { return nb <= 256 ? 256 : (nb + 63) & ~63; }
+
+// Whether it takes a call that gemv_f32act_q4_kernel can take too (rows: the outputs, SwiGLU's of one selection; norm: RMSNORM
+// inside). It reads x and, with norm, takes the ordered sums once for 8 rows and more; against that stand threads without a group
+// where nb does not fill them, and few workgroups where the rows are few. Times in us, gemv_f32act_q4_kernel's first:
+//   norm          4096 x 2080 / 2400 / 4096 / 8192 11.3 / 12.3 / 20.3 / 57 and 8.8 / 9.4 / 11.4 / 20; 14336 x 2080 / 2400 / 2720 / 4096
+//                 13.8 / 15.6 / 17.8 / 36 and 16.0 / 16.7 / 17.6 / 19; 32768 x 2080 27 and 22
+//   norm, SwiGLU  256 x 2080 / 3072 / 3584 9.8 / 12.4 / 14.3 and 12.1 / 13.0 / 14.2; 1024 x 2080 12.7 and 12.2; 8192 x 2080 15.6 and 17.2;
+//                 14336 x 2400 / 2720 / 2752 / 4096 24.9 / 27.3 / 27.0 / 53 and 27.3 / 28.4 / 25.9 / 30; 65536 x 2080 / 2400 62 / 78 and 65 / 69
+//   plain         4096 x 2080 / 3072 / 3584 / 4096 5.4 / 6.0 / 6.7 / 9.0 and 5.8 / 6.1 / 6.3 / 6.6; 576 / 1536 / 6144 / 8192 x 4096 5.6 / 6.4 /
+//                 8.3 / 9.4 and 6.2 / 6.2 / 8.9 / 9.0; 2048 / 3072 / 8192 / 32768 x 4128 (half the threads) 7.5 / 7.3 / 10.2 / 31 and 5.9 / 7.7
+//                 / 12.3 / 41; 4096 / 6144 x 6144 (three quarters) 12.7 / 11.5 and 8.6 / 12.8; 4096 / 14336 x 8192 19 / 38 and 9.4 / 27
+//   SwiGLU        4096 x 2080 / 2720 / 3072 8.2 / 11.3 / 12.1 and 8.9 / 9.5 / 9.3; 14336 x 3072 / 4096 22.0 / 28.7 and 22.4 / 23.9; 256 / 1024 x
+//                 4096 6.8 / 15.6 and 9.2 / 9.4; 8192 / 32768 x 4128 19.5 / 51 and 21.1 / 76
+inline bool f32q4_wide_route(bool swiglu, bool norm, int nb, int64_t rows) {
+  if (norm) {
+    if (!swiglu) return nb >= 80 || rows <= 8192 || rows > 24576;
+    return nb >= 112 || (nb >= 86 && rows >= 512) || (nb >= 75 && rows > 24576) || (rows >= 1024 && rows <= 6144);
+  }
+  const bool full = 100 * f32q4_wide_sets(nb) * nb >= 85 * f32q4_wide_threads(nb);  // 85% of the threads have a group
+  if (nb >= 192) return full || rows <= 4096;
+  if (swiglu) {
+    if (nb >= 128) return rows >= 512 && (full || rows <= 4096);
+    return nb >= 86 && rows >= (nb >= 112 ? 1024 : 2048) && rows <= (full ? 14336 : 4096);
+  }
+  if (nb < 128) return false;
+  return full ? rows >= 1536 && (rows <= 4096 || rows >= 8192) : rows >= 512 && rows <= (nb >= 160 ? 4096 : 2048);
+}
+
 }  // namespace elmh

@@ -2434,7 +2434,7 @@ __global__ __launch_bounds__(256) void gemv_f32act_q4_kernel(const F32Args a) {
   }
 }
 
-// The same for long rows (64 < nb <= 512 groups): a thread keeps its group's 32 x values in registers and takes the group's
+// The same for long rows (64 < nb <= 512 groups, f32q4_wide_route): a thread keeps its group's 32 x values in registers and takes the group's
 // items of 8 consecutive rows (128 contiguous bytes; of gate and of up with SW), all requested at the start, so that a
 // workgroup (nb threads, or S * nb where several fit 256) reads x once for 8 S rows and not once per 1 or 2. x is requested
 // before the weights: RMSNORM's sums run while those are in flight, once per workgroup: the launch makes about two
@@ -2442,10 +2442,7 @@ __global__ __launch_bounds__(256) void gemv_f32act_q4_kernel(const F32Args a) {
 // workgroup: 36 against 30 us for gate and up with RMSNORM inside). The ordered sums at both ends (RMSNORM's 1024 adds, the
 // fold) are what is left above the memory time: gate and up 2 x 14336 x 4096 55 -> 30 us, down 4096 x 14336 47 -> 16 us
 // (73 and 37 MB of weights).
-constexpr int kF32QRows = 8;
 typedef float v4flu __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned is enough
-inline bool f32q4_wide_ok(int nb, int H) { return nb > 64 && nb <= 512 && H >= kF32QRows && H % kF32QRows == 0; }
-inline int f32q4_wide_sets(int nb) { return nb <= 256 ? 256 / nb : 1; }
 template <bool SW>
 __global__ __launch_bounds__(512) void gemv_f32act_q4_wide_kernel(const F32Args a) {
   extern __shared__ __align__(16) float f32q4w_lds[];
@@ -3527,10 +3524,17 @@ static int f32q4_tile_rows(int H, int nb, int nsel, int rows) {
   return rt;
 }
 
+// The q4 GEMV of one token: which of its two kernels takes the call, or neither
+enum class F32Q4 { kNone, kGroups, kWide };  // -, gemv_f32act_q4_kernel, gemv_f32act_q4_wide_kernel
+static F32Q4 f32q4_kernel(int T, int K, int nb, int H, int nsel, int rows, bool norm) {
+  if (T != 1 || K != nb * kBlock) return F32Q4::kNone;
+  const bool groups = H >= 1 && !(H & (H - 1)) &&
+                      f32q4_lds_bytes(K, nb, f32q4_tile_rows(H, nb, nsel, rows), nsel, norm) <= kMaxLds - 1024;
+  if (f32q4_wide_ok(nb, H) && (!groups || f32q4_wide_route(nsel == 2, norm, nb, rows))) return F32Q4::kWide;
+  return groups ? F32Q4::kGroups : F32Q4::kNone;
+}
 bool f32act_q4_ok(int T, int K, int nb, int H, int nsel, int rows, bool norm) {
-  if (T == 1 && K == nb * kBlock && f32q4_wide_ok(nb, H)) return true;
-  return T == 1 && H >= 1 && !(H & (H - 1)) && K == nb * kBlock &&
-         f32q4_lds_bytes(K, nb, f32q4_tile_rows(H, nb, nsel, rows), nsel, norm) <= kMaxLds - 1024;
+  return f32q4_kernel(T, K, nb, H, nsel, rows, norm) != F32Q4::kNone;
 }
 
 hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s) {
@@ -3538,9 +3542,10 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
   const int n = swiglu ? 1 : a.n_targets;
   int rows = 0;
   for (int i = 0; i < n; ++i) rows += a.tg[i].N;
-  if (a.T == 1 && dtype == WQ4 && f32act_q4_ok(a.T, a.K, a.nb, a.H, nsel, rows, a.nw != nullptr)) {
+  const F32Q4 q4 = dtype == WQ4 ? f32q4_kernel(a.T, a.K, a.nb, a.H, nsel, rows, a.nw != nullptr) : F32Q4::kNone;
+  if (q4 != F32Q4::kNone) {
     F32Args b = a;
-    if (f32q4_wide_ok(a.nb, a.H)) {
+    if (q4 == F32Q4::kWide) {
       const int S = b.rt = f32q4_wide_sets(a.nb), pst = (((a.nb + 3) >> 2) | 1) << 2;
       int tiles = 0;
       for (int i = 0; i < n; ++i) {
@@ -3549,7 +3554,7 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
       }
       b.tile_start[n] = tiles;
       if (tiles < 1) return hipErrorInvalidValue;
-      const int threads = a.nb <= 256 ? 256 : (a.nb + 63) & ~63;
+      const int threads = f32q4_wide_threads(a.nb);
       const size_t lds = ((size_t)nsel * S * kF32QRows * pst + (a.nw ? 4 * (size_t)norm_rowlen(a.K) : 0)) * sizeof(float);
       if (swiglu) b.tile_start[1] = tiles;
       // about two workgroups per CU, each with the same number of tiles (the last ones perhaps one fewer)

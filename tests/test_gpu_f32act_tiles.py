@@ -108,3 +108,45 @@ def test_f32act_long_row_gemv(ctx, shape):
             b.free()
     for d in dws + [du]:
         d.free()
+
+
+# (rows of each target, K, RMSNORM inside, SwiGLU): several tiles per workgroup (more than 512 tiles), the last workgroups with one
+# fewer, targets whose boundary a workgroup crosses between two of its tiles; 1, 2 and 3 row sets, 256 threads and more
+TILED = [((4200, 1003, 40), 4128, True, False), ((24600, 100), 2080, True, False), ((8300,), 2752, True, True), ((8311,), 4096, False, True),
+         ((8200, 4100, 16), 4096, False, False), ((4130, 8), 10272, False, False), ((4100,), 8192, True, True)]
+
+
+@pytest.mark.parametrize("case", TILED, ids=["x".join(map(str, c[0] + (c[1],))) for c in TILED])
+def test_f32act_long_row_gemv_several_tiles_a_workgroup(ctx, case):
+    rows, k, norm, sw = case
+    r = np.random.default_rng(rows[0] + k)
+
+    def w(n):
+        return O.make_weight(r.standard_normal((n, k), dtype=np.float32) * np.float32(0.05), O.Q4)
+
+    ws = [w(n) for n in rows] + ([w(rows[0])] if sw else [])
+    dws = [up(ctx, v) for v in ws]
+    x = r.normal(0, 1, (1, k)).astype(np.float32)
+    nw = r.normal(1, 0.1, k).astype(np.float32)
+    xin = O.rmsnorm(x, nw, 1e-5) if norm else x
+    bx, bn = ctx.buffer(x.nbytes).upload(x), ctx.buffer(nw.nbytes).upload(nw)
+    by = [ctx.buffer(4 * n) for n in rows]
+    print(f"[gpu] f32act long rows, several tiles: {case}", flush=True)
+    if sw:
+        if norm:
+            ctx.rmsnorm_swiglu_dev(bx.ptr, bn.ptr, 1e-5, 1, k, dws[0], dws[1], by[0].ptr, act=E.ACT_F32)
+        else:
+            ctx.swiglu_dev(bx.ptr, 1, k, dws[0], dws[1], by[0].ptr, act=E.ACT_F32)
+        want = [O.cpu_swiglu(xin, ws[0], ws[1], act_quant=False)]
+    else:
+        if norm:
+            ctx.rmsnorm_matmul_dev(bx.ptr, bn.ptr, 1e-5, 1, k, dws, [b.ptr for b in by], None, act=E.ACT_F32)
+        else:
+            ctx.matmul_dev(bx.ptr, 1, k, dws, [b.ptr for b in by], None, act=E.ACT_F32)
+        want = O.cpu_matmul(xin, ws, None, act_quant=False)
+    for b, v in zip(by, want):
+        assert bits_equal(b.download(v.shape, np.float32), v)
+    for b in [bx, bn] + by:
+        b.free()
+    for d in dws:
+        d.free()

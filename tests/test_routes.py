@@ -21,6 +21,7 @@ extern "C" int split16(int q8, int sw, int tok, int ring, int nb, int T, long wg
   return gemm_split16_route(q8 != 0, sw != 0, tok != 0, ring != 0, nb, T, wgs);
 }
 extern "C" int f32gemm(int q8, int sw, int T, int K, const int* N, int n) { return (int)f32_gemm_route(q8 != 0, sw != 0, T, K, N, n); }
+extern "C" int q4wide(int sw, int norm, int nb, long rows) { return f32q4_wide_route(sw != 0, norm != 0, nb, rows); }
 """
 STEP, ROWS4, ROWS8, PREFILL64, PREFILL, DECODE64, WHOLE, GLOBAL = range(8)
 
@@ -145,3 +146,22 @@ def test_f32_gemm_tiles(routes):
     for k, T, n, pairs in [(64, 33, 4096, 1), (64, 93, 1536, 1), (64, 64, 512, 0), (64, 256, 4096, 0), (96, 33, 4096, 0)]:
         assert (f32gemm(routes, n, k, T) == R64X2) == bool(pairs), (n, k, T)
     assert f32gemm(routes, 65536 * 64, 32, 2) != R64X2  # more row groups than a grid's second dimension takes
+
+
+# (SwiGLU, norm): (rows, K, faster with a group per thread and 8 rows each?), measured on both sides
+WIDE = {
+    (0, 1): [(4096, 2080, 1), (14336, 2080, 0), (14336, 2400, 0), (14336, 2720, 1), (32768, 2080, 1), (16, 4096, 1), (14336, 4096, 1)],
+    (1, 1): [(256, 2080, 0), (1024, 2080, 1), (8192, 2080, 0), (256, 3072, 0), (576, 3072, 1), (256, 3584, 1), (14336, 2720, 0),
+             (14336, 2752, 1), (14336, 4096, 1), (65536, 2080, 0), (32768, 2400, 1)],
+    (0, 0): [(4096, 2080, 0), (65536, 2080, 0), (4096, 3072, 0), (576, 4096, 0), (1536, 4096, 1), (4096, 4096, 1), (6144, 4096, 0),
+             (8192, 4096, 1), (14336, 4096, 1), (2048, 4128, 1), (3072, 4128, 0), (32768, 4128, 0), (4096, 6144, 1), (6144, 6144, 0),
+             (16, 8192, 1), (14336, 8192, 1), (6144, 8224, 0), (4096, 14336, 1)],
+    (1, 0): [(14336, 2080, 0), (256, 4096, 0), (1024, 4096, 1), (4096, 3072, 1), (14336, 4096, 1), (8192, 4128, 0), (32768, 4128, 0),
+             (4096, 14336, 1)],
+}
+
+
+@pytest.mark.parametrize("kind", WIDE, ids=lambda k: f"{'swiglu' if k[0] else 'plain'}{'-norm' * k[1]}")
+def test_f32_one_token_long_rows_where_they_are_faster(routes, kind):
+    for n, k, wide in WIDE[kind]:
+        assert bool(routes.q4wide(*kind, k // 32, C.c_long(n))) == bool(wide), (n, k)
