@@ -207,6 +207,16 @@ inline F32Gemm f32_gemm_route(bool q8, bool swiglu, int T, int K, const int* N, 
   return wgs(32, 16) >= (swiglu ? 384 : 256) ? F32Gemm::k32x16 : F32Gemm::k16x8;
 }
 
+// gemm_f32act_tile_kernel's workgroups as a grid: kF32GridX to a row of it (a dispatch counts threads per dimension in 32 bits, and
+// a workgroup has 512), the last row perhaps not full. False: more than a grid holds.
+constexpr int kF32GridX = 1 << 22;
+inline bool f32_gemm_grid(int64_t wgs, unsigned* x, unsigned* y) {
+  if (wgs < 1 || wgs > INT32_MAX) return false;
+  *x = (unsigned)(wgs < kF32GridX ? wgs : kF32GridX);
+  *y = (unsigned)((wgs + kF32GridX - 1) / kF32GridX);
+  return true;
+}
+
 // ---------------------------------------------------------------- f32-activation q4 GEMV (one token)
 
 // gemv_f32act_q4_wide_kernel: nb groups per row spread over a workgroup's threads (256 up to 256 groups, which then hold several

@@ -2941,8 +2941,10 @@ __global__ __launch_bounds__(64 * kF32TWaves) void gemm_f32act_tile_kernel(const
   constexpr int NW = (WSL + NT - 1) / NT, NX = (XSL + NT - 1) / NT;
   __shared__ __align__(16) v4fl wl[2][NSEL][P][R * 4], xl[2][P][TT * 4];
   const int tt = a.rt;  // token tiles: consecutive workgroups share their weight rows
-  int grp = blockIdx.x / tt;
-  const int t0 = (blockIdx.x - grp * tt) * TT;
+  const int wg = blockIdx.y * kF32GridX + blockIdx.x;  // below 2^31 (f32_gemm_grid)
+  int grp = wg / tt;
+  if (blockIdx.y > 0 && grp >= a.tile_start[a.n_targets]) return;  // past the last, in the grid's last row (the whole workgroup)
+  const int t0 = (wg - grp * tt) * TT;
   const GemvTarget tg = f32_target<SW>(a, grp);
   const int K = a.K, K4 = K & ~3, H = a.H, nb = a.nb, T = a.T;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -3656,8 +3658,9 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
       }
       b.tile_start[n] = groups;
       b.rt = (a.T + kF32TWaves * TX - 1) / (kF32TWaves * TX);
-      if (groups < 1 || (int64_t)groups * b.rt > INT32_MAX) return hipErrorInvalidValue;
-      const int grid = groups * b.rt, threads = 64 * kF32TWaves;
+      dim3 grid;
+      if (!f32_gemm_grid((int64_t)groups * b.rt, &grid.x, &grid.y)) return hipErrorInvalidValue;
+      const int threads = 64 * kF32TWaves;
       if constexpr (RY <= 2) {
         if (swiglu) {
           if (dtype == WQ8) gemm_f32act_tile_kernel<WQ8, true, RY, TX, P><<<grid, threads, 0, s>>>(b);

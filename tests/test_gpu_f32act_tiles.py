@@ -150,3 +150,26 @@ def test_f32act_long_row_gemv_several_tiles_a_workgroup(ctx, case):
         b.free()
     for d in dws:
         d.free()
+
+
+def test_f32act_gemm_more_workgroups_than_a_grid_row(ctx):
+    """One row and 67 million tokens as SwiGLU: 4.2 million workgroups of 512 threads, more than one dimension of a grid is given
+    (2^22), the last grid row not full. x repeats a pattern of tokens, so every token's output is known."""
+    k, pat, T = 4, 1 << 20, 16 * ((1 << 22) + 37) - 3
+    r = np.random.default_rng(8)
+    wg, wu = weight(r, 1, k, O.Q8), weight(r, 1, k, O.Q8)
+    dg, du = up(ctx, wg), up(ctx, wu)
+    x = r.normal(0, 1, (pat, k)).astype(np.float32)
+    bx, by = ctx.buffer(T * k * 4), ctx.buffer(T * 4)
+    bx.upload(x)
+    for t in range(pat, T, pat):
+        ctx.memcpy_d2d(bx.ptr + t * k * 4, bx.ptr, min(pat, T - t) * k * 4)
+    print(f"[gpu] f32act gemm of {T} tokens", flush=True)
+    ctx.swiglu_dev(bx.ptr, T, k, dg, du, by.ptr, act=E.ACT_F32)
+    got = by.download((T,), np.float32).view(np.int32)
+    want = O.cpu_swiglu(x, wg, wu, act_quant=False).ravel().view(np.int32)
+    for t in range(0, T, pat):
+        assert np.array_equal(got[t:t + pat], want[:min(pat, T - t)]), t
+    for b in (bx, by):
+        b.free()
+    dg.free(), du.free()
