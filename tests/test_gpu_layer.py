@@ -126,8 +126,9 @@ def test_attention_past_lds_score_rows(ctx, shape):
 @pytest.mark.parametrize("rope", [False, True])
 def test_attention_long_cache_decode_steps(ctx, rope):
     """Decode steps with the position read from device memory (the form a captured graph replays) over a
-    cache of 16,384 positions, whose score row the step kernel keeps whole in LDS (more than 64 KB: the
-    kernel's LDS limit is raised to gfx950's 160 KB), at positions around the 320-position value chunks."""
+    cache of 16,384 positions, whose score row attention_step_kernel keeps whole in LDS (128 KB with its key
+    pieces, past the head-size-64 kernel's: the limit is raised to gfx950's 160 KB), at the first positions
+    and past 64-position pieces; the chunks between run on the head-size-64 chunk kernel."""
     nh, nkv, hd, mc = 9, 3, 64, 16384
     r = np.random.default_rng(77 + int(rope))
     tab = O.rope_table(hd, mc, 100000.0) if rope else None
