@@ -94,8 +94,9 @@ inline AttnKernel attention_route(const AttnCall& c) {
   // Longer chunks: attention_rows_kernel, at head size 64 from 4096 (token, head) pairs on (9 heads: 512 tokens 31 against
   // 48 us with attention_prefill64_kernel, 128 tokens 11 against 8.4; 32 heads, 64 tokens at 600 positions 34 against 32).
   // R = 8 rows a workgroup read the keys half as often as 4; 4 fill the chip at fewer rows and keep more workgroups per CU
-  // where the score rows are long (32 heads of size 128: 256 tokens at 256 positions 80 against 86 us; 128 tokens 19.5
-  // against 17.4; 512 at 1500 986 against 613).
+  // where the score rows are long (32 heads of size 128 over 8 kv heads, 4 and 8 rows: 96 / 128 / 256 / 320 tokens at 256 positions
+  // 34 / 40 / 76 / 100 and 39 / 41 / 71 / 90 us; 256 at 600 / 1500 131 / 277 and 121 / 268, 384 at 600 / 1500 205 / 401 and 203 / 648,
+  // 512 at 1500 / 3000 545 / 1296 and 898 / 1605).
   auto groups = [&](int R) { return ((int64_t)c.T * grp + R - 1) / R; };
   const int R = c.n_kv * groups(8) >= 1024 && 3 * attention_rows_lds_bytes(8, c.hd, c.n_cap) <= kMaxLds ? 8 : 4;
   if (!fuse && !c.pos_dev && c.aligned && groups(R) < 65536 && (c.hd != 64 || pairs >= 4096) &&
@@ -207,14 +208,12 @@ inline F32Gemm f32_gemm_route(bool q8, bool swiglu, int T, int K, const int* N, 
   return wgs(32, 16) >= (swiglu ? 384 : 256) ? F32Gemm::k32x16 : F32Gemm::k16x8;
 }
 
-// gemm_f32act_tile_kernel's workgroups as a grid: kF32GridX to a row of it (a dispatch counts threads per dimension in 32 bits, and
-// a workgroup has 512), the last row perhaps not full. False: more than a grid holds.
-constexpr int kF32GridX = 1 << 22;
-inline bool f32_gemm_grid(int64_t wgs, unsigned* x, unsigned* y) {
-  if (wgs < 1 || wgs > INT32_MAX) return false;
-  *x = (unsigned)(wgs < kF32GridX ? wgs : kF32GridX);
-  *y = (unsigned)((wgs + kF32GridX - 1) / kF32GridX);
-  return true;
+// Token tiles of one launch of gemm_f32act_tile_kernel over `groups` row groups: a dispatch counts a dimension's threads in 32 bits,
+// and a workgroup has 512. 0: more row groups than one grid takes. (The token range of a launch costs nothing; a second grid
+// dimension in the kernel took 0.3 us of 15.)
+inline int f32_gemm_tiles_per_launch(int64_t groups) {
+  constexpr int64_t kMost = int64_t(1) << 22;
+  return groups < 1 ? 0 : (int)(kMost / groups);
 }
 
 // ---------------------------------------------------------------- f32-activation q4 GEMV (one token)

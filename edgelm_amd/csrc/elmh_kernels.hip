@@ -19,6 +19,7 @@
 #include "elm_dma.h"
 #include "elm_sum.h"
 
+#include <algorithm>
 #include <cstring>
 #include <type_traits>
 
@@ -2941,10 +2942,8 @@ __global__ __launch_bounds__(64 * kF32TWaves) void gemm_f32act_tile_kernel(const
   constexpr int NW = (WSL + NT - 1) / NT, NX = (XSL + NT - 1) / NT;
   __shared__ __align__(16) v4fl wl[2][NSEL][P][R * 4], xl[2][P][TT * 4];
   const int tt = a.rt;  // token tiles: consecutive workgroups share their weight rows
-  const int wg = blockIdx.y * kF32GridX + blockIdx.x;  // below 2^31 (f32_gemm_grid)
-  int grp = wg / tt;
-  if (blockIdx.y > 0 && grp >= a.tile_start[a.n_targets]) return;  // past the last, in the grid's last row (the whole workgroup)
-  const int t0 = (wg - grp * tt) * TT;
+  int grp = blockIdx.x / tt;
+  const int t0 = (blockIdx.x - grp * tt) * TT;
   const GemvTarget tg = f32_target<SW>(a, grp);
   const int K = a.K, K4 = K & ~3, H = a.H, nb = a.nb, T = a.T;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -3657,20 +3656,34 @@ hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s)
         groups += (a.tg[i].N + 16 * RY - 1) / (16 * RY);
       }
       b.tile_start[n] = groups;
-      b.rt = (a.T + kF32TWaves * TX - 1) / (kF32TWaves * TX);
-      dim3 grid;
-      if (!f32_gemm_grid((int64_t)groups * b.rt, &grid.x, &grid.y)) return hipErrorInvalidValue;
-      const int threads = 64 * kF32TWaves;
-      if constexpr (RY <= 2) {
-        if (swiglu) {
-          if (dtype == WQ8) gemm_f32act_tile_kernel<WQ8, true, RY, TX, P><<<grid, threads, 0, s>>>(b);
-          else gemm_f32act_tile_kernel<WQ4, true, RY, TX, P><<<grid, threads, 0, s>>>(b);
-          return hipGetLastError();
+      // one launch, or several over ranges of the tokens where its workgroups would be more than a grid takes
+      const int tiles = f32_gemm_tiles_per_launch(groups), threads = 64 * kF32TWaves, TT = kF32TWaves * TX;
+      if (tiles < 1) return hipErrorInvalidValue;
+      for (int64_t t0 = 0; t0 < a.T; t0 += (int64_t)tiles * TT) {
+        b.T = (int)std::min<int64_t>(a.T - t0, (int64_t)tiles * TT);
+        b.rt = (b.T + TT - 1) / TT;
+        b.x = a.x + t0 * a.K;
+        for (int i = 0; i < n; ++i) {
+          b.tg[i].y = a.tg[i].y + t0 * a.tg[i].N;
+          b.tg[i].res = a.tg[i].res ? a.tg[i].res + t0 * a.tg[i].N : nullptr;
         }
+        const int grid = groups * b.rt;
+        bool done = false;
+        if constexpr (RY <= 2) {
+          if (swiglu) {
+            if (dtype == WQ8) gemm_f32act_tile_kernel<WQ8, true, RY, TX, P><<<grid, threads, 0, s>>>(b);
+            else gemm_f32act_tile_kernel<WQ4, true, RY, TX, P><<<grid, threads, 0, s>>>(b);
+            done = true;
+          }
+        }
+        if (!done) {
+          if (dtype == WQ8) gemm_f32act_tile_kernel<WQ8, false, RY, TX, P><<<grid, threads, 0, s>>>(b);
+          else gemm_f32act_tile_kernel<WQ4, false, RY, TX, P><<<grid, threads, 0, s>>>(b);
+        }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
       }
-      if (dtype == WQ8) gemm_f32act_tile_kernel<WQ8, false, RY, TX, P><<<grid, threads, 0, s>>>(b);
-      else gemm_f32act_tile_kernel<WQ4, false, RY, TX, P><<<grid, threads, 0, s>>>(b);
-      return hipGetLastError();
+      return hipSuccess;
     };
     using std::integral_constant;
     switch (route) {

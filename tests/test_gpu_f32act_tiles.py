@@ -152,9 +152,9 @@ def test_f32act_long_row_gemv_several_tiles_a_workgroup(ctx, case):
         d.free()
 
 
-def test_f32act_gemm_more_workgroups_than_a_grid_row(ctx):
-    """One row and 67 million tokens as SwiGLU: 4.2 million workgroups of 512 threads, more than one dimension of a grid is given
-    (2^22), the last grid row not full. x repeats a pattern of tokens, so every token's output is known."""
+def test_f32act_gemm_more_workgroups_than_a_grid(ctx):
+    """One row and 67 million tokens as SwiGLU: 4.2 million workgroups of 512 threads, more than one launch is given (2^22), so a
+    second one takes the last 589 tokens. x repeats a pattern of tokens, so every token's output is known."""
     k, pat, T = 4, 1 << 20, 16 * ((1 << 22) + 37) - 3
     r = np.random.default_rng(8)
     wg, wu = weight(r, 1, k, O.Q8), weight(r, 1, k, O.Q8)

@@ -21,7 +21,7 @@ extern "C" int split16(int q8, int sw, int tok, int ring, int nb, int T, long wg
   return gemm_split16_route(q8 != 0, sw != 0, tok != 0, ring != 0, nb, T, wgs);
 }
 extern "C" int f32gemm(int q8, int sw, int T, int K, const int* N, int n) { return (int)f32_gemm_route(q8 != 0, sw != 0, T, K, N, n); }
-extern "C" int f32grid(long wgs, unsigned* x, unsigned* y) { return f32_gemm_grid(wgs, x, y); }
+extern "C" int f32tiles(long groups) { return f32_gemm_tiles_per_launch(groups); }
 extern "C" int q4wide(int sw, int norm, int nb, long rows) { return f32q4_wide_route(sw != 0, norm != 0, nb, rows); }
 """
 STEP, ROWS4, ROWS8, PREFILL64, PREFILL, DECODE64, WHOLE, GLOBAL = range(8)
@@ -168,13 +168,11 @@ def test_f32_one_token_long_rows_where_they_are_faster(routes, kind):
         assert bool(routes.q4wide(*kind, k // 32, C.c_long(n))) == bool(wide), (n, k)
 
 
-def test_f32_gemm_grid_holds_every_workgroup(routes):
-    """A dispatch counts threads per dimension in 32 bits: 512 a workgroup. Every workgroup has its place, up to 2^31 - 1."""
-    x, y = C.c_uint(), C.c_uint()
-    for wgs in (1, 2, 511, 1 << 22, (1 << 22) + 1, 8388607, 8388608, 8388609, 123456789, (1 << 31) - 1):
-        assert routes.f32grid(C.c_long(wgs), C.byref(x), C.byref(y))
-        assert x.value * 512 < 1 << 32 and 1 <= y.value <= 65535
-        assert (y.value - 1) * x.value < wgs <= y.value * x.value
-        assert y.value == 1 or x.value == 1 << 22
-    for wgs in (0, -1, 1 << 31):
-        assert not routes.f32grid(C.c_long(wgs), C.byref(x), C.byref(y))
+def test_f32_gemm_launches_fit_a_grid(routes):
+    """A dispatch counts threads per dimension in 32 bits: 512 a workgroup. Up to the rows that the kernel before took (65,535
+    groups of 64, which are 262,140 of 16) at least one token tile fits."""
+    for groups in (1, 2, 3, 511, 65535, 262140, (1 << 22) - 1, 1 << 22):
+        tiles = routes.f32tiles(C.c_long(groups))
+        assert tiles >= 1 and tiles * groups * 512 < 1 << 32 and (tiles + 1) * groups > 1 << 22
+    for groups in (0, -5, (1 << 22) + 1, 1 << 31):
+        assert routes.f32tiles(C.c_long(groups)) == 0
