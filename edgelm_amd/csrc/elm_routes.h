@@ -138,8 +138,8 @@ constexpr int kLds16MaxBlocks = 48;  // gemm_lds16_kernel: rows of at most this 
 //   SwiGLU q8, per block  (82 KB of LDS: one workgroup per CU) 14336 x 4096 at 16 (896): 31.7, 45.3; 11008 x 4096 at 16 (688): 30.3,
 //                         35.1; 8192 x 4096 at 16 (512) 0.85; 2048 x 2048 at 64 / 65 (512 / 640) 0.96 / 1.26; 1536 x 1568 at 48 (288 of
 //                         49 blocks): 15.1, 15.8
-// More tokens over few rows fill the chip with the other's workgroups earlier (256 x 2048 q8 at 1536 tokens, 1536 workgroups 1.08; as
-// SwiGLU q4 at 1024 tokens, 1024 workgroups 1.05). The ring kernel, which serves what makes 128 tiles of 128 rows x 64 tokens, is
+// More tokens over few rows fill the chip with the other's workgroups earlier (256 x 2048 q8 at 1536 tokens, 1536 workgroups 1.08, 256 x
+// 4096 0.92; as SwiGLU q4 256 x 2048 / 4096 at 1024 tokens, 1024 workgroups 1.05 / 1.03). The ring kernel, which serves what makes 128 tiles of 128 rows x 64 tokens, is
 // slower at few tokens: 16384 x 4096 at 16 tokens (1024 workgroups) 0.52 q4, 0.65 q8, SwiGLU 0.26 and 0.48; 32000 x 4096 at 16
 // (2000) 0.84 and 1.06, per token 0.76 and 1.00.
 inline bool gemm_split16_route(bool q8, bool swiglu, bool token, bool ring, int nb, int T, int64_t wgs) {
@@ -147,10 +147,10 @@ inline bool gemm_split16_route(bool q8, bool swiglu, bool token, bool ring, int 
   const int64_t load = wgs * ((nb + 15) / 16 * 16) / nb;
   const bool many = T > (q8 && token ? 1024 : 768);
   if (swiglu) {
-    if (q8 && !token && !ring) return load <= (many || nb < 64 ? 340 : 530);
-    return load <= (many ? 900 : q8 && token ? 1536 : 1200);
+    if (q8 && !token && !ring) return load <= (nb < 64 || (many && nb < 128) ? 340 : 530);
+    return load <= (many ? (nb < 128 ? 900 : 1100) : q8 && token ? 1536 : 1200);
   }
-  if (many) return load <= 1200;
+  if (many) return load <= (q8 && nb < 128 ? 1200 : 1600);
   if (q8) return load <= (!token ? 1840 : ring ? 1900 : 2100);
   return load <= (!token || ring || nb >= 256 ? 2100 : nb >= 96 ? 1840 : 1700);
 }

@@ -88,9 +88,9 @@ def test_attention_short_prompts_append_inside(routes, nh, nkv):
 # the two kernels cross; the rows of a 16 x 16 tile grid counted in eights
 SPLIT = {
     (0, 0, 0): [(4096, 14336, 16, 1), (4096, 14336, 128, 1), (4096, 14336, 256, 0), (8192, 2048, 64, 1), (8192, 2048, 65, 0),
-                (1536, 1568, 320, 0), (64, 2048, 4096, 0), (32000, 4096, 16, 1)],
+                (1536, 1568, 320, 0), (64, 2048, 4096, 0), (256, 4096, 1536, 1), (32000, 4096, 16, 1)],
     (1, 0, 0): [(4096, 4096, 112, 1), (4096, 4096, 128, 0), (2048, 2048, 192, 1), (2048, 2048, 256, 0), (32000, 4096, 8, 0),
-                (16384, 4096, 16, 1), (128, 1568, 2048, 0), (1024, 14336, 512, 0)],
+                (16384, 4096, 16, 1), (128, 1568, 2048, 0), (256, 2048, 1536, 0), (256, 4096, 1536, 1), (1024, 14336, 512, 0)],
     (0, 0, 1): [(1536, 1568, 192, 1), (1536, 1568, 224, 0), (8192, 2048, 64, 0), (1024, 4096, 512, 0), (4096, 14336, 128, 1),
                 (32000, 4096, 16, 1)],
     (1, 0, 1): [(4096, 14336, 128, 1), (16384, 4096, 32, 0), (256, 2048, 1536, 0), (4096, 4096, 256, 0)],
