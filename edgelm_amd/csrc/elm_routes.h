@@ -182,6 +182,8 @@ enum class F32Gemm { k64x2, k16x8, k32x16, k64x16, k64x32 };
 //   5, 6       24576 x 256 8.2 and 8.8, x 576 15.8 and 13.6
 //   8          49152 x 64 / 160 / 192 8.4 / 12.0 / 14.5 and 11.2 / 14.7 / 15.2
 //   17         16384 x 192 11.2 and 12.2, 49152 x 192 as SwiGLU 56 and 62 (a second tile of one token)
+//   9 to 33    with a quarter of the 16-token tiles empty, 49152 x 32 at 12 / 24 / 33 as SwiGLU q8 15.5 / 29 / 41 and 20 / 39 / 52; without
+//              (16, 32) 49152 x 64 30 and 22 at 16
 //   K = 64     4096 x 33 tokens 5.1 and 6.0, 1536 x 93 5.0 and 5.8; 512 x 64 3.9 and 3.4, 4096 x 128 10.1 and 9.0
 inline F32Gemm f32_gemm_route(bool q8, bool swiglu, int T, int K, const int* N, int n) {
   auto groups = [&](int rows) {
@@ -197,9 +199,8 @@ inline F32Gemm f32_gemm_route(bool q8, bool swiglu, int T, int K, const int* N, 
   else if (T <= 4) pair = K <= (many || !swiglu ? 640 : 384) || rows > 98304;
   else if (T <= 6) pair = K <= (swiglu ? 128 : 256);
   else if (T <= 8) pair = K <= (swiglu ? 96 : 192);
-  else if (T <= 12) pair = K <= 64 && !swiglu;
   else if (T > 16 && T <= 20) pair = swiglu ? K <= (many ? 320 : 192) : !many && K <= 192;
-  else if (T <= 24) pair = K <= 64 && !many && !swiglu;
+  else if (T <= 40) pair = K <= 64 && 4 * T <= 48 * ((T + 15) / 16) && (swiglu || !many || T <= 12);
   if (pair && groups(64) <= 65535) return F32Gemm::k64x2;
   auto wgs = [&](int r, int t) { return groups(r) * ((T + t - 1) / t); };
   if (T <= (K < 2048 ? 6 : 5)) return !swiglu && wgs(64, 16) >= 512 ? F32Gemm::k64x16 : F32Gemm::k16x8;

@@ -1111,7 +1111,7 @@ __global__ __launch_bounds__(256) void attention_prefill64_kernel(
 //    rows over two pairs of waves where two waves cover the dims); values come straight from the cache, 16 positions per
 //    batch, the next batch in flight; p_j = e_j * inv of 16 positions lies in 16 lanes and is broadcast by the multiply. Where
 //    all of a batch's positions are below nmax a load is one instruction, the row's offset in a scalar register (with a clamped
-//    address each: 256 tokens at 256 positions 76 us against 73, 512 at 1500 580 against 538).
+//    address each: 256 tokens at 256 positions 73.6 us against 69.6 with the append, 512 at 1500 580 against 538).
 //    Positions that only some of the rows see are masked (a later token's value may be anything), the others are not.
 // 32 heads over 8 kv heads, head size 128, 256 tokens at 256 cached positions: 70 us with the append against 800 us with one workgroup per
 // (token, head) (attention_kernel), which read the keys and values again for every row and ran each row's chains on one wave.

@@ -146,6 +146,8 @@ def test_f32_gemm_tiles(routes):
     assert f32gemm(routes, 1536, 576, 93, q8=1, sw=1) == R16X8 and f32gemm(routes, 4096, 4096, 64, sw=1) == R32X16
     for k, T, n, pairs in [(64, 33, 4096, 1), (64, 93, 1536, 1), (64, 64, 512, 0), (64, 256, 4096, 0), (96, 33, 4096, 0)]:
         assert (f32gemm(routes, n, k, T) == R64X2) == bool(pairs), (n, k, T)
+    for T, pairs in [(9, 1), (12, 1), (16, 0), (24, 1), (32, 0), (33, 1), (48, 0)]:
+        assert (f32gemm(routes, 16384, 64, T, sw=1) == R64X2) == bool(pairs), T
     assert f32gemm(routes, 65536 * 64, 32, 2) != R64X2  # more row groups than a grid's second dimension takes
 
 
