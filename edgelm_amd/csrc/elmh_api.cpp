@@ -1316,9 +1316,11 @@ int elmh_attention_dev(elmh_ctx* c, const float* q, const float* k, const float*
   if (rc) return rc;
   DeviceGuard g(c);
   float* gsc = nullptr;
-  // one token: the rows that the same step takes with its position in device memory (sized for the whole cache), so that a
-  // step captured after one that ran op by op finds them
-  const AttnCall call = attention_call(T, pos0, T == 1, n_heads, n_kv, head_dim, k_cache, max_ctx, false);
+  // one token, outside a capture: also the rows that the same step takes with its position in device memory (sized for the
+  // whole cache), so that a step captured after one that ran op by op finds them. This call does not need them.
+  const AttnCall step = attention_call(1, 0, true, n_heads, n_kv, head_dim, k_cache, max_ctx, false);
+  if (T == 1 && attention_global_score_bytes(step) > c->asc.cap && !capturing(c)) (void)attention_scores(c, step, &gsc);
+  const AttnCall call = attention_call(T, pos0, false, n_heads, n_kv, head_dim, k_cache, max_ctx, false);
   if (const int r2 = attention_scores(c, call, &gsc)) return r2;
   HIP_OR_FAIL(c, launch_attention(q, k, v, out, T, pos0, nullptr, n_heads, n_kv, head_dim, k_cache, v_cache, max_ctx,
                                   rope_cos, rope_sin, c->stream, nullptr, nullptr, 0, nullptr, gsc));
