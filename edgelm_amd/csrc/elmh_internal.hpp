@@ -158,9 +158,9 @@ bool gemm_qf_ok(int dtype, int T, int nb, int H, int N, int64_t rows_pad);
 hipError_t launch_gemv_a8(int dtype, int swiglu, const GemvArgs& a, int total_tiles, hipStream_t s);
 hipError_t launch_gemm_a8(int dtype, int swiglu, int token_mode, const GemmArgs& a, int total_tiles, hipStream_t s);
 hipError_t launch_f32act(int dtype, int swiglu, const F32Args& a, hipStream_t s);
-// True if launch_f32act runs the group-parallel q4 GEMV for this call (one token, q4 targets of tile
-// height H, `rows` output rows, nsel = 2 for SwiGLU): its LDS, sized for the tile height the launch
-// picks and, with norm (RMSNORM applied to x inside, a.nw), for the squares, fits a workgroup.
+// True if launch_f32act runs a q4 GEMV of its own for this call (one token, q4 targets of tile height H, `rows` output rows, nsel = 2
+// for SwiGLU; with norm, RMSNORM applied to x inside, a.nw): gemv_f32act_q4_kernel, whose LDS, sized for the tile height the launch
+// picks and for norm's squares, fits a workgroup, or gemv_f32act_q4_wide_kernel (f32q4_wide_route).
 bool f32act_q4_ok(int T, int K, int nb, int H, int nsel, int rows, bool norm);
 hipError_t launch_silu_mul(const float* g, const float* u, float* y, int64_t n, hipStream_t s);
 // The non-matmul ops of a layer (elmh_layer.hip), same float order as edgelm's cpu backend.
