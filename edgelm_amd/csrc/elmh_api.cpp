@@ -639,7 +639,10 @@ int norm_to_scratch(elmh_ctx* c, const float* x, const float* nw, float eps, int
 }
 
 struct DeviceGuard {
-  explicit DeviceGuard(elmh_ctx* c) { (void)hipSetDevice(c->device); }
+  explicit DeviceGuard(elmh_ctx* c) {
+    (void)hipSetDevice(c->device);
+    call_device = c->device;
+  }
 };
 
 constexpr int kArgStepMaxN = 64 * 4096;  // launch_argmax_parts: 64 workgroups of 4096 values

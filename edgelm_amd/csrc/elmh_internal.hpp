@@ -165,10 +165,12 @@ bool f32act_q4_ok(int T, int K, int nb, int H, int nsel, int rows, bool norm);
 hipError_t launch_silu_mul(const float* g, const float* u, float* y, int64_t n, hipStream_t s);
 // The non-matmul ops of a layer (elmh_layer.hip), same float order as edgelm's cpu backend.
 hipError_t launch_rmsnorm(const float* x, const float* w, float* y, int rows, int dim, float eps, hipStream_t s);
-// The dynamic-LDS limit of `kernel` raised to `bytes` on the current device, at its first call there (once: the kernel's own)
+// The device of the call on this thread: every entry point that launches makes its context's device current and says so here
+// (asking the runtime at each launch instead takes 56 ns of the host)
+inline thread_local int call_device = 0;
+// The dynamic-LDS limit of `kernel` raised to `bytes` on the call's device, at its first call there (once: the kernel's own)
 inline bool raise_dynamic_lds(DeviceOnce& once, const void* kernel, size_t bytes) {
-  int device = 0;
-  const bool ok = hipGetDevice(&device) == hipSuccess && once.run(device, [&] {
+  const bool ok = once.run(call_device, [&] {
     return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
   });
   if (!ok) (void)hipGetLastError();  // the caller takes another kernel or reports it: no later launch does

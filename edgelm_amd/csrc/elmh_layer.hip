@@ -1849,7 +1849,7 @@ static hipError_t launch_attention_rows(const float* q, float* out, const float*
   return hipGetLastError();
 }
 
-// the attention kernels keep a whole score row (and a chunk of values) in LDS: allow them up to kMaxAttnLds on the current
+// the attention kernels keep a whole score row (and a chunk of values) in LDS: allow them up to kMaxAttnLds on the call's
 // device
 bool raise_lds_limit() {
   const void* kernels[] = {(const void*)attention_kernel<64, false>, (const void*)attention_kernel<0, false>,
@@ -1888,8 +1888,7 @@ hipError_t launch_attention(const float* q, const float* k, const float* v, floa
   const float* kn = fuse ? k : nullptr;
   const float* vn = fuse ? v : nullptr;
   static DeviceOnce raised;
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess || !raised.run(device, raise_lds_limit)) return hipErrorInvalidValue;
+  if (!raised.run(call_device, raise_lds_limit)) return hipErrorInvalidValue;
   if (route == AttnKernel::kStep) {
     const dim3 grid(n_kv, grp, T);
     const size_t lds = attention_step_lds_bytes(hd, n_cap);
